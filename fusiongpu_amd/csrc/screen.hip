@@ -12,9 +12,9 @@
 // Here no LUT is built.  Instead:
 //   1. Threshold.  For every query, its first usable probed list is screened
 //      with upper bounds U(v) >= d(q, v) of the exact distances.  The list's
-//      vectors fall into 32 groups by position; the k-th smallest of the 32
-//      group minima of U is T(q): k distinct vectors have d <= T(q), so the
-//      final k-th distance is <= T(q).
+//      vectors fall into groups by position (64 for k <= 32, else 128); the
+//      k-th smallest of the group minima of U is T(q): k distinct vectors have
+//      d <= T(q), so the final k-th distance is <= T(q).
 //   2. Screen.  Every probed list whose lower bound (list_lower_bound, the
 //      flow kernel's rule) is <= T(q) is screened with lower bounds
 //      L(v) <= d(q, v) in the form V(v) = L(v) - T(q) <= 0: a vector with
@@ -454,9 +454,8 @@ __global__ __launch_bounds__(256) void screen_pairs1_kernel(ScreenArgs a) {
   if (lane == 0) a.first[q] = f;
 }
 
-// Round 2 pairs, one wave a query.  First T(q): the k-th smallest of the 32
-// group minima of U over the query's first list (the minimum, over the list's
-// chunks, of each chunk's per-group minimum), taken back from the round-1
+// Round 2 pairs, one wave a query.  First T(q): the k-th smallest of the
+// group minima of U over the query's first list, taken back from the round-1
 // row's scale 2^-t to the data's scale 2^S and inflated by 1 + 2^-14; +inf
 // without a round-1 pair or with fewer than k groups holding a value
 // (FLT_MAX, and nothing more, for the queries whose candidates are set).  Then
@@ -485,11 +484,19 @@ __global__ __launch_bounds__(256) void screen_pairs2_kernel(ScreenArgs a) {
   // Every chunk's group minima load goes out with the first pair's record
   // (a chain of the two is the kernel's longest latency); the query's block
   // holds kMaxChunks x kMaxGroups words, those past its chunks are unused.
+  // A chunk holds 32 groups for k <= 32: its even chunks go to lanes 0-31, the
+  // odd ones to lanes 32-63.
+  const bool wide = screen_groups(a.k) == 64;
   uint32_t gc[kMaxChunks];
   {
-    const uint32_t* g = a.gminbuf + (size_t)q * kMaxChunks * kMaxGroups + lane;
+    const uint32_t* g = a.gminbuf + (size_t)q * kMaxChunks * kMaxGroups;
+    if (wide) {
 #pragma unroll
-    for (int c = 0; c < kMaxChunks; ++c) gc[c] = g[c * kMaxGroups];
+      for (int c = 0; c < kMaxChunks; ++c) gc[c] = g[c * kMaxGroups + lane];
+    } else {
+#pragma unroll
+      for (int c = 0; c < kMaxChunks / 2; ++c) gc[c] = g[(2 * c + (lane >> 5)) * kMaxGroups + (lane & 31)];
+    }
   }
   const int2 f = a.first[q];
   const int ft = f.y & 0xFF;  // the round-1 row scale exponent
@@ -499,14 +506,37 @@ __global__ __launch_bounds__(256) void screen_pairs2_kernel(ScreenArgs a) {
     if (lane == 0) a.thr[q] = FLT_MAX;
     return;
   }
-  uint32_t gm = 0x7F800000u;
-  if (f.x >= 0 && lane < screen_groups(a.k)) {
+  // The groups: the even and the odd chunks of a list apart, 64 groups in one
+  // wave vector (k <= 32) or 128 in two.  The rank of T(q) in its list is
+  // that of the k-th first-hit group, ln(1 - k / G) / ln(1 - 1 / G): with one
+  // group per lane column (G = 32, or 64 above k = 32) it is 12 for k = 10 but
+  // 129 for k = 32, 97 for k = 50 and 303 for k = 64; with twice the groups 11,
+  // 44, 63 and 88.  A further doubling (73 for k = 64) costs two more wave sorts.
+  // Measured, one group per lane column before: 2000 queries, 128 probes, k 64
+  // over 1M x 128 at 64 subspaces 6.88 -> 1.73 ms (candidates halved, 1174 ->
+  // 206 queries past the candidate buffer); the 10k-query pruned scan over 10M x
+  // 96 with limit_k 50 1.506 -> 1.460 ms; k = 10 unchanged (0.332 ms).
+  uint32_t gm = 0x7F800000u, gm2 = 0x7F800000u;
+  if (f.x >= 0) {
     const int nch = f.y >> 8;
+    if (wide) {
 #pragma unroll
-    for (int c = 0; c < kMaxChunks; ++c) gm = min(gm, c < nch ? gc[c] : 0x7F800000u);
+      for (int c = 0; c < kMaxChunks; c += 2) {
+        gm = min(gm, c < nch ? gc[c] : 0x7F800000u);
+        gm2 = min(gm2, c + 1 < nch ? gc[c + 1] : 0x7F800000u);
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < kMaxChunks / 2; ++c) gm = min(gm, 2 * c + (lane >> 5) < nch ? gc[c] : 0x7F800000u);
+    }
   }
   // U >= 0, so float order is unsigned order of the bits
   wave_sort_u32(gm);
+  if (wide && (f.y >> 8) > 1) {
+    wave_sort_u32(gm2);
+    gm = min(gm, (uint32_t)wave_reverse((int)gm2));
+    bitonic_pass_u32<64>(gm, true);
+  }
   const float kth = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)gm, a.k - 1));
   // the group minima are at the round-1 row's scale 2^-t
   const float T = kth < INFINITY ? f_above(ldexp((double)kth, ft) * kTInfl) : INFINITY;

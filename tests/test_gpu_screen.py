@@ -306,3 +306,25 @@ def test_screen_k_above_32_uses_64_groups(k):
     st = _check(idx, q, cent, cb, offs, ids, codes, 8, k)
     assert st["queries_with_threshold"] == 90 and st["pairs_round1"] == 90
     idx.close()
+
+
+@pytest.mark.parametrize("k", [1, 31, 32, 33, 64])
+def test_screen_threshold_groups_at_chunk_edges(k):
+    """The threshold's groups split a first list's even and odd chunks (256 vectors; longer past eight chunks):
+    lists of one partial chunk up to more than eight, each the first list of several queries."""
+    _say(f"screen threshold groups, k {k}")
+    rng = np.random.default_rng(100 + k)
+    dim, m = 128, 32
+    lens = np.array([64, 255, 256, 257, 511, 513, 769, 2047, 2049, 4100])
+    offs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n = int(offs[-1])
+    ids = rng.permutation(n).astype(np.int32)
+    codes = rng.integers(0, 256, (n, m), dtype=np.uint8)
+    cent = rng.uniform(-1, 1, (lens.size, dim)).astype(np.float32)
+    cb = (rng.standard_normal((m, 256, dim // m)) * 0.1).astype(np.float32)
+    idx = fg.Index.from_arrays(dim, m, offs, ids, codes, cent, cb)
+    assert idx.screen_ready
+    q = np.repeat(cent, 7, axis=0) + (rng.standard_normal((7 * lens.size, dim)) * 0.1).astype(np.float32)
+    st = _check(idx, q.astype(np.float32), cent, cb, offs, ids, codes, 3, k)
+    assert st["queries_with_threshold"] == 7 * lens.size and st["queries_to_lut_kernel"] <= 7 * lens.size // 4
+    idx.close()
