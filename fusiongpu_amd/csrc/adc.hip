@@ -266,17 +266,134 @@ __global__ __launch_bounds__(kNT) void adc_plain_kernel(AdcArgs a) {
   plain_query<D, M>(a, (int)blockIdx.x, smem, s_thr);
 }
 
-// The generic kernel over the queries a.qlist[0 .. *a.qcount): the exact LUT
-// path for the queries the MFMA screen hands back.  A persistent grid; with
-// an empty list every workgroup ends at once.
+// The exact LUT path for the queries the MFMA screen hands back,
+// a.qlist[0 .. *a.qcount), on a persistent grid (with an empty list every
+// workgroup ends at once).  A handed query is rare and alone, so its probes are
+// split over the idle workgroups: S = grid / count parts (at most what the
+// query's part of the workspace can hold), part j walking probes j, j + S, ....
+// Every part starts from the query's bound key (the screen's rescore leaves
+// the key after the k-th best of the candidates it did keep, kNoThr without
+// any; a key must be below it to enter), skips
+// the lists whose lower bound exceeds it, and shares the running k-th key with
+// the other parts through that key in global memory (a 64-bit atomic min; a
+// stale value only skips less).  The last part to arrive merges the parts'
+// sorted keys.  Measured on C2 shapes (8 handed queries of 10,000, 32
+// probes): 106 us with one workgroup a query and no bound, 32 us now; 206 of
+// 2000 queries at 128 probes and 64 subspaces: about 1.4 ms, 64 us now.
+constexpr int kHandProbes = 256;  // probes a query can have (the coarse step's limit)
+
 template <int D, int M>
-__global__ __launch_bounds__(kNT) void adc_plain_list_kernel(AdcArgs a) {
+__device__ __forceinline__ void hand_part(const AdcArgs& a, int q, int part, int S, float* smem,
+                                          unsigned long long& s_thr, int* s_list, float* s_lb, int& s_next,
+                                          int& s_last) {
+  using C = Cfg<D, M>;
+  constexpr int G = kNT / kPQK;  // threads sharing one codeword
+  constexpr int MG = M / G;      // subspaces per thread
+  float* r = smem + C::R_OFF;
+  float* qs = smem + C::Q_OFF;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kc = tid & (kPQK - 1), g = tid / kPQK;
+  const int k = a.k;
+  unsigned long long* gthr = reinterpret_cast<unsigned long long*>(a.hand + (size_t)q * a.hand_stride);
+  int* garr = reinterpret_cast<int*>(gthr + 1);
+  for (int i = tid; i < D; i += kNT) qs[i] = a.queries[(size_t)(q / a.qdiv) * D + i];
+  // This part's probes: list (-1: pruned, out of range or empty) and bound.
+  const int np = part < a.nprobe ? (a.nprobe - part + S - 1) / S : 0;
+  for (int i = tid; i < np; i += kNT) {
+    const size_t t = (size_t)q * a.nprobe + part + (size_t)i * S;
+    const uint32_t l = a.probes[t];
+    const bool use = l < (uint32_t)a.nlist && a.offsets[l + 1] > a.offsets[l];
+    s_list[i] = use ? (int)l : -1;
+    s_lb[i] = use && a.list_skip && a.probe_dists ? list_lower_bound(a.probe_dists[t], a.rmax[l]) : 0.0f;
+  }
+  if (tid == 0) s_thr = kNoThr;
+
+  uint64_t lk = kPadKey;
+  uint64_t own = kNoThr;
+  uint4 w0[C::NV4], w1[C::NV4];
+  int i0 = kPadId, i1 = kPadId;
+  for (int at = 0;;) {
+    __syncthreads();  // the last scan's LUT reads and s_thr updates, the tables
+    if (wave == 0) {
+      // Exchange the running k-th key, then the next list it does not rule out.
+      uint64_t t = s_thr;
+      if (lane == 0) {
+        const uint64_t o = atomicMin(gthr, (unsigned long long)t);
+        t = o < t ? o : t;
+        s_thr = t;
+      }
+      t = readlane64(t, 0);
+      const float thr_hi = __uint_as_float((uint32_t)(t >> 32)) * (1.0f + 0x1p-16f);
+      int nx = np;
+      for (int b = at; b < np; b += kWave) {
+        const uint64_t m = __ballot(b + lane < np && s_list[b + lane] >= 0 && !(s_lb[b + lane] > thr_hi));
+        if (m) {
+          nx = b + (__ffsll((unsigned long long)m) - 1);
+          break;
+        }
+      }
+      if (lane == 0) s_next = nx;
+    }
+    __syncthreads();
+    const int i = s_next;
+    if (i >= np) break;
+    at = i + 1;
+    const int l = s_list[i];
+    const int start = a.offsets[l];
+    const int n = a.offsets[l + 1] - start;
+    // First-round code loads go out before the LUT build, which hides their latency.
+    load_pair<M>(a.codes, a.vec_ids, start, n, wave * kVecPerWaveRound + lane, w0, w1, i0, i1);
+    if (tid < D) r[tid] = qs[tid] - a.centroids[(size_t)l * D + tid];
+    __syncthreads();
+#pragma unroll
+    for (int mm = 0; mm < MG; ++mm) {
+      const int m = g * MG + mm;
+      float rr[C::S], cb[C::S];  // a part scans few lists: the codebook (L2) is not kept in registers
+      load_row<C::S>(a.codebook + ((size_t)m * kPQK + kc) * C::S, cb);
+#pragma unroll
+      for (int j = 0; j < C::S; ++j) rr[j] = r[m * C::S + j];
+      smem[m * kPQK + kc] = lut_entry<C::S>(rr, cb);
+    }
+    __syncthreads();
+    scan_list<D, M, 0, kNW, false>(smem, a.codes, a.vec_ids, start, n, k, wave, w0, w1, i0, i1, lk, own, &s_thr);
+  }
+
+  uint64_t* mk = reinterpret_cast<uint64_t*>(smem);
+  mk[wave * kWave + lane] = lk;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll 1
+  for (int w = 1; w < kNW; ++w) wave_merge_sorted64_k(lk, mk[w * kWave + lane]);
+  if (S > 1) {
+    uint64_t* parts = a.hand_keys + (size_t)q * a.hand_keys_stride;
+    if (lane < k) parts[(size_t)part * k + lane] = lk;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (lane == 0) s_last = __hip_atomic_fetch_add(garr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
+    wave_lds_sync();
+    if (!s_last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll 1
+    for (int j = 0; j < S; ++j)
+      if (j != part) wave_merge_sorted64_k(lk, lane < k ? parts[(size_t)j * k + lane] : kPadKey);
+  }
+  write_topk(lk, q, k, a);
+}
+
+template <int D, int M>
+__global__ __launch_bounds__(kNT) void adc_hand_kernel(AdcArgs a) {
   __shared__ __align__(16) float smem[Cfg<D, M>::SMEM];
   __shared__ unsigned long long s_thr;
+  __shared__ int s_list[kHandProbes];
+  __shared__ float s_lb[kHandProbes];
+  __shared__ int s_next, s_last;
   const int count = min(*a.qcount, a.nq);
-  for (int i = (int)blockIdx.x; i < count; i += (int)gridDim.x) {
-    const int q = a.qlist[i];
-    if (q >= 0 && q < a.nq) plain_query<D, M>(a, q, smem, s_thr);
+  if (count <= 0) return;
+  const int fit = (int)min((long long)a.nprobe, a.hand_keys_stride / a.k);  // parts a query's region holds
+  const int S = max(1, min(fit, (int)gridDim.x / count));
+  for (long long it = blockIdx.x; it < (long long)count * S; it += gridDim.x) {
+    const int q = a.qlist[it / S];
+    if (q >= 0 && q < a.nq)
+      hand_part<D, M>(a, q, (int)(it % S), S, smem, s_thr, s_list, s_lb, s_next, s_last);
     __syncthreads();
   }
 }
@@ -821,14 +938,13 @@ fgpu_status launch_plain(const AdcArgs& a, hipStream_t s) {
 }
 
 template <int D, int M>
-fgpu_status launch_plain_list(const AdcArgs& a, hipStream_t s) {
+fgpu_status launch_hand(const AdcArgs& a, hipStream_t s) {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  // Few workgroups: the list is usually empty, and then each ends at once.
-  const int grid = std::max(1, std::min(a.nq, cus / 4));
-  hipLaunchKernelGGL((adc_plain_list_kernel<D, M>), dim3((unsigned)grid), dim3(kNT), 0, s, a);
+  const int grid = (int)std::min<int64_t>((int64_t)a.nq * a.nprobe, cus);
+  hipLaunchKernelGGL((adc_hand_kernel<D, M>), dim3((unsigned)grid), dim3(kNT), 0, s, a);
   FGPU_HIP(hipGetLastError());
   return FGPU_OK;
 }
@@ -869,15 +985,17 @@ fgpu_status launch_adc_plain(int dim, int m, const AdcArgs& a, hipStream_t s) {
   return set_error(FGPU_ERR_UNSUPPORTED, "adc: unsupported (dim, pq_m)");
 }
 
-fgpu_status launch_adc_plain_list(int dim, int m, const AdcArgs& a, hipStream_t s) {
-  FGPU_CHECK(a.k >= 1 && a.k <= 64 && a.qlist && a.qcount, FGPU_ERR_ARG, "adc: bad query list launch");
+fgpu_status launch_adc_hand(int dim, int m, const AdcArgs& a, hipStream_t s) {
+  FGPU_CHECK(a.k >= 1 && a.k <= 64 && a.qlist && a.qcount && a.hand && a.hand_keys && a.nprobe >= 1 &&
+                 a.nprobe <= kHandProbes,
+             FGPU_ERR_ARG, "adc: bad query list launch");
   if (a.nq <= 0) return FGPU_OK;
-  if (dim == 128 && m == 32) return launch_plain_list<128, 32>(a, s);
-  if (dim == 128 && m == 16) return launch_plain_list<128, 16>(a, s);
-  if (dim == 128 && m == 64) return launch_plain_list<128, 64>(a, s);
-  if (dim == 96 && m == 48) return launch_plain_list<96, 48>(a, s);
-  if (dim == 96 && m == 32) return launch_plain_list<96, 32>(a, s);
-  if (dim == 96 && m == 16) return launch_plain_list<96, 16>(a, s);
+  if (dim == 128 && m == 32) return launch_hand<128, 32>(a, s);
+  if (dim == 128 && m == 16) return launch_hand<128, 16>(a, s);
+  if (dim == 128 && m == 64) return launch_hand<128, 64>(a, s);
+  if (dim == 96 && m == 48) return launch_hand<96, 48>(a, s);
+  if (dim == 96 && m == 32) return launch_hand<96, 32>(a, s);
+  if (dim == 96 && m == 16) return launch_hand<96, 16>(a, s);
   return set_error(FGPU_ERR_UNSUPPORTED, "adc: unsupported (dim, pq_m)");
 }
 

@@ -663,9 +663,8 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
     sa.events = ev ? ev + 2 : nullptr;
     FGPU_TRY(launch_screen(ix->dim, ix->m, sa, s));
     AdcArgs a = adc_args(ix, dq, nq, pid, pd, nprobe, k, d_out_ids, d_out_dists);
-    a.qlist = sw.flist;
-    a.qcount = sw.zero + kCtrFlag;
-    FGPU_TRY(launch_adc_plain_list(ix->dim, ix->m, a, s));
+    screen_hand(sa, &a);
+    FGPU_TRY(launch_adc_hand(ix->dim, ix->m, a, s));
     FGPU_HIP(mark(kStageEvents - 1));
     return FGPU_OK;
   }
@@ -890,9 +889,8 @@ fgpu_status two_phase(const fgpu_index* ix, const float* dq, int nq, const uint3
             FGPU_TRY(launch_screen(ix->dim, ix->m, sa, s));
             AdcArgs la = adc_args(ix, cq, nvq, tw.vprobe, tw.vpd, 1, limit_k, tw.vids, tw.vd);
             la.qdiv = p1;
-            la.qlist = tw.sw.flist;
-            la.qcount = tw.sw.zero + kCtrFlag;
-            FGPU_TRY(launch_adc_plain_list(ix->dim, ix->m, la, s));
+            screen_hand(sa, &la);
+            FGPU_TRY(launch_adc_hand(ix->dim, ix->m, la, s));
             // single-probe mode: both rounds screen the sp_cnt pairs
             FGPU_TRY(launch_tp_stats(sa.cand_cnt, sa.thr, nvq, kScreenCandCap, tw.sw.zero + kCtrFlag, tw.sp_cnt,
                                      tw.sp_cnt, tw.boff, ix->d_offsets, ix->nlist, d_stats, s));

@@ -94,10 +94,18 @@ struct AdcArgs {
   // in *qctr (the select's side write).  The launch skips its own reset when
   // it equals the grid it launches (flow_grid).
   int qctr_preset = 0;
-  // launch_adc_plain_list only: the queries to search, qlist[0 .. *qcount)
-  // (device memory; the count is read on the device).
+  // launch_adc_hand only: the queries to search, qlist[0 .. *qcount) (device
+  // memory; the count is read on the device); per query q, hand[q hand_stride]:
+  // a 64-bit key above every member of its top-k (kPadKey: none known) and an
+  // arrival count (0); and room for the parts' keys at
+  // hand_keys[q hand_keys_stride].  The screen's rescore writes the first
+  // three; the keys live where its pair records were.
   const int* qlist = nullptr;
   const int* qcount = nullptr;
+  uint32_t* hand = nullptr;
+  long long hand_stride = 0;
+  uint64_t* hand_keys = nullptr;
+  long long hand_keys_stride = 0;
 };
 // Id written to every slot of a query whose result a bounded-wait give-up may
 // have touched (the reference's padding id is -1; it never writes -2).
@@ -111,9 +119,9 @@ bool adc_supported(int dim, int m);
 fgpu_status launch_list_radius(const float* codebook, int m, int sub, const uint8_t* codes, const int32_t* offsets,
                                int nlist, float* rmax, hipStream_t s);
 fgpu_status launch_adc_plain(int dim, int m, const AdcArgs& a, hipStream_t s);
-// The generic (one workgroup a query, every probed list) kernel over the
-// queries a.qlist[0 .. *a.qcount), on a persistent grid.
-fgpu_status launch_adc_plain_list(int dim, int m, const AdcArgs& a, hipStream_t s);
+// The queries a.qlist[0 .. *a.qcount) that the screen hands back: their probes
+// split over a persistent grid, bounded by what the screen found (a.hand).
+fgpu_status launch_adc_hand(int dim, int m, const AdcArgs& a, hipStream_t s);
 // The grid of the flow-kernel launch launch_adc_plain makes for these sizes
 // (the start value of its query counter), or 0 if that call takes another
 // kernel.
@@ -200,8 +208,10 @@ int64_t screen_gmin_words(int nq);
 fgpu_status launch_screen_prep(const float* codebook, int m, int sub, int scale_exp, const uint8_t* codes,
                                int64_t total, uint16_t* cb16, uint4* vext, unsigned int* xmax_bits, hipStream_t s);
 // Threshold, screen and rescore; the queries it cannot answer are listed in
-// flist[0 .. ctr[kCtrFlag]) for launch_adc_plain_list.
+// flist[0 .. ctr[kCtrFlag]) for launch_adc_hand, whose hand-over fields
+// screen_hand sets (they reuse buffers the screen is done with).
 fgpu_status launch_screen(int dim, int m, const ScreenArgs& a, hipStream_t s);
+void screen_hand(const ScreenArgs& sa, AdcArgs* a);
 
 // ---- twophase.hip --------------------------------------------------------------
 struct TwoPhaseArgs {

@@ -47,6 +47,27 @@ __device__ __forceinline__ float lut_entry(const float* r, const float* p) {
   }
 }
 
+// S consecutive floats (a codeword, a centroid's sub-vector) in the widest loads S allows.
+template <int S>
+__device__ __forceinline__ void load_row(const float* p, float (&v)[S]) {
+  if constexpr (S % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < S / 4; ++i) {
+      const float4 t = reinterpret_cast<const float4*>(p)[i];
+      v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+    }
+  } else if constexpr (S % 2 == 0) {
+#pragma unroll
+    for (int i = 0; i < S / 2; ++i) {
+      const float2 t = reinterpret_cast<const float2*>(p)[i];
+      v[2 * i] = t.x; v[2 * i + 1] = t.y;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < S; ++i) v[i] = p[i];
+  }
+}
+
 template <int M>
 __device__ __forceinline__ void load_codes(const uint8_t* __restrict__ codes, int64_t vec, uint4 (&w)[M / 16]) {
   const uint4* p = reinterpret_cast<const uint4*>(codes + vec * M);

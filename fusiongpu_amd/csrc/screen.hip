@@ -987,26 +987,6 @@ __global__ __launch_bounds__(kSW * kWave) void screen_kernel(ScreenArgs a) {
 }
 
 // ---- exact rescore ------------------------------------------------------------------------
-template <int S>
-__device__ __forceinline__ void load_row(const float* p, float (&v)[S]) {
-  if constexpr (S % 4 == 0) {
-#pragma unroll
-    for (int i = 0; i < S / 4; ++i) {
-      const float4 t = reinterpret_cast<const float4*>(p)[i];
-      v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
-    }
-  } else if constexpr (S % 2 == 0) {
-#pragma unroll
-    for (int i = 0; i < S / 2; ++i) {
-      const float2 t = reinterpret_cast<const float2*>(p)[i];
-      v[2 * i] = t.x; v[2 * i + 1] = t.y;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < S; ++i) v[i] = p[i];
-  }
-}
-
 // One wave a query: the exact ADC distance of every candidate in the
 // reference's direct form (the LUT entry's chain per subspace, summed in
 // ascending m), then the k smallest (distance, id) keys.  A persistent grid
@@ -1019,6 +999,7 @@ __device__ __forceinline__ void load_row(const float* p, float (&v)[S]) {
 // the query's one list, so the residual r = fl(q - c) is formed once in LDS
 // (the same fp32 subtraction) instead of loading the centroid per candidate.
 constexpr int kRW = 16;  // waves per rescore workgroup
+constexpr int kHandStride = kMaxChunks * kMaxGroups;  // words a query of gminbuf, free again after round 2's pairs
 template <int D, int M, bool ONE>
 __global__ __launch_bounds__(kRW * kWave) void rescore_kernel(ScreenArgs a) {
   constexpr int S = D / M;
@@ -1038,13 +1019,24 @@ __global__ __launch_bounds__(kRW * kWave) void rescore_kernel(ScreenArgs a) {
     if (i + stride < a.nq) qn = a.order ? a.order[i + stride] : i + stride;  // the next query's index, early
     const float T = a.thr[q];
     const int cnt = __builtin_amdgcn_readfirstlane(a.cand_cnt[q]);
-    if (!(T < INFINITY) || cnt > a.cand_cap) {
+    // Handed to the LUT kernel: a query without a threshold at once, one with
+    // more candidates than fit after the rescore of those that did: its top-k
+    // lies below the key after their k-th (cand_cap >= k vectors).
+    const bool over = cnt > a.cand_cap;
+    auto hand = [&](uint64_t bound) {
       if (lane == 0) {
+        uint32_t* h = a.gminbuf + (size_t)q * kHandStride;
+        *reinterpret_cast<uint64_t*>(h) = bound;
+        h[2] = 0u;
         const int f = atomicAdd(&a.ctr[kCtrFlag], 1);
         a.flist[f] = q;
       }
+    };
+    if (!(T < INFINITY)) {
+      hand(kPadKey);
       continue;
     }
+    const int ncand = over ? a.cand_cap : cnt;
     if constexpr (ONE) {
       const uint32_t l1 = a.probes[q];  // cnt > 0 only when it is a usable list
       for (int d = lane; d < D; d += kWave)
@@ -1055,10 +1047,10 @@ __global__ __launch_bounds__(kRW * kWave) void rescore_kernel(ScreenArgs a) {
     wave_sync();
     const float* qv = qs[wave];
     uint64_t lk = kPadKey;
-    for (int i0 = 0; i0 < cnt; i0 += kWave) {
+    for (int i0 = 0; i0 < ncand; i0 += kWave) {
       const int i = i0 + lane;
       uint64_t key = kPadKey;
-      if (i < cnt) {
+      if (i < ncand) {
         const uint2 e = a.cand[(size_t)q * a.cand_cap + i];
         const int64_t pos = e.x;
         const float* cen = a.centroids + (size_t)(ONE ? 0 : e.y) * D;
@@ -1094,7 +1086,9 @@ __global__ __launch_bounds__(kRW * kWave) void rescore_kernel(ScreenArgs a) {
       else
         wave_merge_sorted64_k(lk, key);
     }
-    if (lane < a.k) {
+    if (over) {
+      hand(readlane64(lk, a.k - 1) + 1);  // the k-th itself may be the answer's k-th
+    } else if (lane < a.k) {
       const int id = key_id(lk);
       const bool pad = id == kPadId;
       a.out_ids[(size_t)q * a.k + lane] = pad ? -1 : id;
@@ -1162,6 +1156,15 @@ fgpu_status launch_screen_prep(const float* codebook, int m, int sub, int scale_
                        scale_exp, codes, total, vext, xmax_bits);
   FGPU_HIP(hipGetLastError());
   return FGPU_OK;
+}
+
+void screen_hand(const ScreenArgs& sa, AdcArgs* a) {
+  a->qlist = sa.flist;
+  a->qcount = sa.ctr + kCtrFlag;
+  a->hand = sa.gminbuf;
+  a->hand_stride = kHandStride;
+  a->hand_keys = reinterpret_cast<uint64_t*>(sa.arec);
+  a->hand_keys_stride = (long long)sa.nprobe * kRec * (long long)(sizeof(uint4) / sizeof(uint64_t));
 }
 
 fgpu_status launch_screen(int dim, int m, const ScreenArgs& a, hipStream_t s) {

@@ -328,3 +328,27 @@ def test_screen_threshold_groups_at_chunk_edges(k):
     st = _check(idx, q.astype(np.float32), cent, cb, offs, ids, codes, 3, k)
     assert st["queries_with_threshold"] == 7 * lens.size and st["queries_to_lut_kernel"] <= 7 * lens.size // 4
     idx.close()
+
+
+@pytest.mark.parametrize("dim,m,k,nq,nprobe", [(128, 32, 32, 300, 6), (128, 16, 1, 3, 1), (128, 64, 64, 1, 37),
+                                               (96, 48, 7, 40, 37), (128, 32, 10, 2, 37)])
+def test_screen_handed_queries_split_their_probes(dim, m, k, nq, nprobe):
+    """Queries handed to the LUT kernel, from more queries than workgroups (one part a query) down to one (a
+    part a probe): lists of tied codes overflow the candidate buffer, and the first queries' nearest list is shorter
+    than k (no bound; for k 1, nothing is).  Lists are empty, short, one chunk and long; ties go by id."""
+    _say(f"handed queries dim={dim} m={m} k={k} nq={nq} nprobe={nprobe}")
+    rng = np.random.default_rng(dim + m + k + nq)
+    lens = np.concatenate([[max(k - 1, 0), 900, 0, 1, 128, 1500], rng.integers(500, 900, 34)])
+    offs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n = int(offs[-1])
+    ids = rng.permutation(n).astype(np.int32)
+    codes = np.repeat(rng.integers(0, 256, (1, m), dtype=np.uint8), n, axis=0)
+    codes[::3] = rng.integers(0, 256, (codes[::3].shape[0], m), dtype=np.uint8)
+    cent = (rng.standard_normal((lens.size, dim)) * 0.05).astype(np.float32)
+    cb = (rng.standard_normal((m, 256, dim // m)) * 0.1).astype(np.float32)
+    idx = fg.Index.from_arrays(dim, m, offs, ids, codes, cent, cb)
+    q = cent[np.arange(nq) % 2] + (rng.standard_normal((nq, dim)) * 1e-3).astype(np.float32)
+    st = _check(idx, q.astype(np.float32), cent, cb, offs, ids, codes, nprobe, k)
+    if nprobe > 1:
+        assert st["queries_to_lut_kernel"] >= (nq + 1) // 2
+    idx.close()
