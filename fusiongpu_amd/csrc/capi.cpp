@@ -1051,6 +1051,9 @@ fgpu_status fgpu_l2_topk(const float* dx, int64_t n, const float* dc, int nc, in
   void* est = cv.take<float>((size_t)rows * ld);
   FGPU_TRY(launch_row_norms(dc, nc, dim, cn, s));
   FGPU_TRY(launch_max_reduce(cn, nc, cmax, s));
+  if (p == 1 && assign_takes(dx, n, dc, nc, dim, rest)) {
+    return launch_assign(dx, n, dc, nc, dim, cmax, est, ws_bytes - (size_t)((char*)est - (char*)ws), d_ids, d_dists, s);
+  }
   for (int64_t b0 = 0; b0 < n; b0 += rows) {
     const int64_t nb = std::min<int64_t>(rows, n - b0);
     FGPU_TRY(launch_gemm_est_sel(dx + b0 * dim, nb, dc, nc, dim, cn, cmax, est, ld, s));

@@ -39,6 +39,21 @@ fgpu_status launch_select_exact(const void* est, int64_t ld, int64_t nrows, int 
                                 const float* cn_max, int p, int prune, float prune_ratio,
                                 int32_t* out_ids, float* out_d, hipStream_t s, int* side = nullptr,
                                 int side_val = 0, unsigned long long* stats = nullptr);
+// The nearest column of every row (p = 1) without an estimate matrix
+// (assign.hip): ids and exact distances; ws holds its column tiles and each
+// row's candidates.  assign_takes: whether it applies (dim 32, 64, 96 or 128,
+// 16-byte aligned arrays, at least kAssignMinRows rows, kAssignMinCols to
+// kAssignMaxCols columns, room for 512 rows) rather than the estimate + select
+// pair.  A workgroup walks every column, so below about 64 workgroups (512
+// rows each) the pair, which also splits the columns, is faster.  Measured (us,
+// pair / this, dim 128): 8192 rows 29 / 51 (256 columns) and 92 / 139 (4096);
+// 65,536 rows 120 / 61 and 624 / 158; 262,144 rows 423 / 118 and 2486 / 360;
+// 65,536 rows of 16 columns 87 / 85.
+constexpr int kAssignMinCols = 32, kAssignMaxCols = 4096;
+constexpr int64_t kAssignMinRows = 32768;
+bool assign_takes(const float* x, int64_t n, const float* c, int nc, int dim, size_t ws_bytes);
+fgpu_status launch_assign(const float* x, int64_t n, const float* c, int nc, int dim, const float* cn_max, void* ws,
+                          size_t ws_bytes, int32_t* ids, float* d, hipStream_t s);
 // Exact kNN over one chunk of <= 4096 base rows c (ids id_base + col), merged
 // into the running top-k in ids/d (k <= 128) when accum != 0.
 fgpu_status launch_knn_chunk(const float* est, int64_t ld, int64_t nrows, int ncols, const float* x, const float* c,

@@ -104,6 +104,65 @@ def test_l2_topk_estimate_extremes(case, dim, p, nc):
     assert np.array_equal(_bits(d), _bits(od))
 
 
+@pytest.mark.parametrize("dim,nc,n", [(128, 4096, 32768), (128, 4095, 33281), (96, 129, 33000), (64, 128, 32769),
+                                      (32, 33, 32768), (128, 32, 32900), (96, 1000, 70001)])
+def test_l2_topk_nearest_large_batches(dim, nc, n):
+    """p = 1 from 32768 rows on takes the register-resident fp16 pass; the same rows in slices of 32767 take the
+    estimate + select pair.  Both equal bit for bit (and the oracle on a sample): column counts at the 32-column
+    tile and four-tile stage edges, row counts off the 512-row workgroup, duplicate and near-equal columns (several
+    candidates in one column class), rows far larger and far smaller than the columns, and NaN and infinite rows
+    and columns."""
+    _say(f"l2_topk nearest dim={dim} nc={nc} n={n}")
+    rng = np.random.default_rng(dim + nc + n)
+    c = rng.standard_normal((nc, dim)).astype(np.float32)
+    x = (c[rng.integers(0, nc, n)] + 0.3 * rng.standard_normal((n, dim))).astype(np.float32)
+    if nc > 64:
+        c[64] = c[0]                                 # equal columns of one class
+        c[40] = c[8] * np.float32(1 + 2e-4)          # closer than the margin
+        c[72] = c[8] * np.float32(1 - 2e-4)
+        x[:50], x[50:90] = c[0], c[8]
+    x[100:110] *= np.float32(1e6)
+    x[110:120] *= np.float32(1e-6)
+    x[120] = 0
+
+    def both(x, c):
+        dx, dc = torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda()
+        ids, d = fg.l2_topk(dx, dc, 1)
+        got = _host(ids)[:, 0], _host(d)[:, 0]
+        parts = [fg.l2_topk(dx[b:b + 32767], dc, 1) for b in range(0, n, 32767)]
+        want = [np.concatenate([_host(p[i])[:, 0] for p in parts]) for i in (0, 1)]
+        assert np.array_equal(got[0], want[0])
+        assert np.array_equal(_bits(got[1]), _bits(want[1]))
+        return got
+    ids, d = both(x, c)
+    oid, od = oracle.coarse(x[:600], c, 1, prune_ratio=np.inf)
+    assert np.array_equal(ids[:600].view(np.uint32), oid[:, 0]) and np.array_equal(_bits(d[:600]), _bits(od[:, 0]))
+    x[200, 3], x[201, 5], x[202] = np.nan, np.inf, -np.inf
+    c[2] = np.nan
+    both(x, c)
+    c[1, 0] = np.inf
+    both(x, c)
+
+
+@pytest.mark.parametrize("case", ["offset", "tiny", "large"])
+def test_l2_topk_nearest_extremes(case):
+    """The same pass where its margin is wide against the differences (a common offset 30 times the spread: every
+    column a candidate of every row) and at scales far from 1."""
+    _say(f"l2_topk nearest extremes {case}")
+    rng = np.random.default_rng(len(case))
+    x = rng.standard_normal((32768, 128)).astype(np.float32)
+    c = rng.standard_normal((200, 128)).astype(np.float32)
+    if case == "offset":
+        off = rng.standard_normal(128).astype(np.float32) * np.float32(300.0)
+        x, c = x + off, c + off
+    else:
+        s = np.float32(1e-15 if case == "tiny" else 1e12)
+        x, c = x * s, c * s
+    ids, d = fg.l2_topk(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), 1)
+    oid, od = oracle.coarse(x, c, 1, prune_ratio=np.inf)
+    assert np.array_equal(_host(ids).view(np.uint32), oid) and np.array_equal(_bits(_host(d)), _bits(od))
+
+
 # --------------------------------------------------------------------------- coarse quantizer (A2, A3)
 @pytest.mark.parametrize("case", ["unit", "x300", "sift_like"])
 def test_coarse_margin_stays_tight_at_large_norms(case):
