@@ -72,6 +72,11 @@ __global__ void fill_i32_kernel(int32_t* __restrict__ p, int64_t n) {
   if (i < n) p[i] = 0;
 }
 
+__global__ void add_i32_kernel(int32_t* __restrict__ p, const int32_t* __restrict__ q, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] += q[i];
+}
+
 __global__ void gather_rows_kernel(const float* __restrict__ x, int dim, const int32_t* __restrict__ rows,
                                    int nrows, float* __restrict__ out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -85,6 +90,109 @@ __global__ void gather_rows_kernel(const float* __restrict__ x, int dim, const i
 // atomics): integer addition is associative, so the result does not depend on
 // the order the atomics land, unlike the reference's float atomicAdd
 // (kmeans_gpu.cuh:94-97).
+// Two forms.  kmeans_accumulate_kernel: one 64-bit atomic a coordinate.  From
+// kOrderedMinRows rows on, the rows are first grouped by centre (a histogram, its
+// scan, a scatter of the row numbers; the order within a centre is free), then
+// each wave sums 128 consecutive grouped rows in registers and adds a centre's
+// sums once: 1M rows of 128 dims and 4096 centres 0.90 -> 0.21 ms (128 M
+// atomics before, 1.6 M now; reading the rows once takes 0.1 ms).
+constexpr int kOrdThreads = 1024, kOrdPer = 8;  // rows a workgroup of the grouping kernels: 8192
+constexpr int kOrdSeg = 128;                    // grouped rows a wave sums
+
+// The workgroup's rows per centre in LDS; the rank of this thread's row i
+// (strided by the workgroup size) among them.
+__device__ __forceinline__ void order_local(const int32_t* assign, int64_t row0, int64_t n, int k, int32_t* bins,
+                                            int (&c)[kOrdPer], int (&rank)[kOrdPer]) {
+  for (int b = threadIdx.x; b < k; b += kOrdThreads) bins[b] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kOrdPer; ++i) {
+    const int64_t r = row0 + (int64_t)i * kOrdThreads + threadIdx.x;
+    c[i] = r < n ? assign[r] : -1;
+    rank[i] = (uint32_t)c[i] < (uint32_t)k ? atomicAdd(&bins[c[i]], 1) : -1;
+  }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(kOrdThreads) void order_count_kernel(const int32_t* __restrict__ assign, int64_t n, int k,
+                                                                  int32_t* __restrict__ counts) {
+  extern __shared__ int32_t bins[];
+  int c[kOrdPer], rank[kOrdPer];
+  order_local(assign, (int64_t)blockIdx.x * kOrdThreads * kOrdPer, n, k, bins, c, rank);
+  for (int b = threadIdx.x; b < k; b += kOrdThreads)
+    if (bins[b] > 0) atomicAdd(&counts[b], bins[b]);
+}
+
+// cursor: the exclusive scan of counts, advanced past each centre's rows.
+__global__ __launch_bounds__(kOrdThreads) void order_scatter_kernel(const int32_t* __restrict__ assign, int64_t n,
+                                                                    int k, int32_t* __restrict__ cursor,
+                                                                    int32_t* __restrict__ order) {
+  extern __shared__ int32_t bins[];
+  const int64_t row0 = (int64_t)blockIdx.x * kOrdThreads * kOrdPer;
+  int c[kOrdPer], rank[kOrdPer];
+  order_local(assign, row0, n, k, bins, c, rank);
+  for (int b = threadIdx.x; b < k; b += kOrdThreads) {
+    const int m = bins[b];
+    if (m > 0) bins[b] = atomicAdd(&cursor[b], m);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kOrdPer; ++i)
+    if (rank[i] >= 0) order[bins[c[i]] + rank[i]] = (int32_t)(row0 + (int64_t)i * kOrdThreads + threadIdx.x);
+}
+
+// One wave a segment of kOrdSeg grouped rows, lanes over dimensions (NV of
+// them a lane).  total: the grouped rows (rows whose centre is in range).
+template <int NV>
+__global__ __launch_bounds__(256) void order_sum_kernel(const float* __restrict__ x, const int32_t* __restrict__ total,
+                                                        const int32_t* __restrict__ assign,
+                                                        const int32_t* __restrict__ order, int dim, int shift,
+                                                        unsigned long long* __restrict__ sums) {
+  constexpr int B = 8;  // rows whose loads are in flight together
+  const int lane = threadIdx.x & 63;
+  const int p0 = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * kOrdSeg;
+  const int p1 = min(p0 + kOrdSeg, *total);
+  long long acc[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) acc[j] = 0;
+  int cur = -1;
+  auto flush = [&]() {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if (cur >= 0 && lane + 64 * j < dim)
+        atomicAdd(&sums[(int64_t)cur * dim + lane + 64 * j], (unsigned long long)acc[j]);
+      acc[j] = 0;
+    }
+  };
+  for (int b0 = p0; b0 < p1; b0 += kWave) {
+    // this batch's rows and centres, one a lane
+    const int r_l = b0 + lane < p1 ? order[b0 + lane] : 0;
+    const int c_l = b0 + lane < p1 ? assign[r_l] : -1;
+    const int m = min(kWave, p1 - b0);
+    for (int i0 = 0; i0 < m; i0 += B) {
+      float v[B][NV];
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const float* xr = x + (int64_t)__builtin_amdgcn_readlane(r_l, min(i0 + i, m - 1)) * dim;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[i][j] = lane + 64 * j < dim ? xr[lane + 64 * j] : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        if (i0 + i >= m) break;
+        const int c = __builtin_amdgcn_readlane(c_l, i0 + i);
+        if (c != cur) {
+          flush();
+          cur = c;
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) acc[j] += __float2ll_rn(ldexpf(v[i][j], shift));
+      }
+    }
+  }
+  flush();
+}
+
 __global__ __launch_bounds__(256) void kmeans_accumulate_kernel(
     const float* __restrict__ x, int64_t n, const int32_t* __restrict__ assign, int dim, int shift,
     unsigned long long* __restrict__ sums, int32_t* __restrict__ counts) {
@@ -607,11 +715,52 @@ fgpu_status launch_maxabs(const float* x, int64_t count, float* out, hipStream_t
   return launch_max_reduce(out, 1023, out + 1023, s);
 }
 
+// Grouping scratch: the centres' offsets and chunk counts, and the row order.
+static size_t order_fixed_bytes(int k) { return carve_bytes<int32_t>((size_t)k + 1) + carve_bytes<int32_t>(k) + 256; }
+size_t kmeans_order_bytes(int k, int64_t rows) { return order_fixed_bytes(k) + carve_bytes<int32_t>(rows); }
+
 fgpu_status launch_kmeans_accumulate(const float* x, int64_t n, const int32_t* assign, int k, int dim, int shift,
-                                     unsigned long long* sums, int32_t* counts, hipStream_t s) {
+                                     unsigned long long* sums, int32_t* counts, void* ows, size_t ows_bytes,
+                                     hipStream_t s) {
   FGPU_TRY(launch1d(fill_u64_kernel, (int64_t)k * dim, 256, s, sums, (int64_t)k * dim));
   FGPU_TRY(launch1d(fill_i32_kernel, (int64_t)k, 256, s, counts, (int64_t)k));
-  return launch1d(kmeans_accumulate_kernel, n * dim, 256, s, x, n, assign, dim, shift, sums, counts);
+  const size_t fixed = order_fixed_bytes(k);
+  const int64_t fit = ows && ows_bytes > fixed ? (int64_t)((ows_bytes - fixed) / sizeof(int32_t)) : 0;
+  if (n < kOrderedMinRows || k > kOrderedMaxCentres || dim > 256 || fit < std::min<int64_t>(n, kOrderedMinRows))
+    return launch1d(kmeans_accumulate_kernel, n * dim, 256, s, x, n, assign, dim, shift, sums, counts);
+  Carve cv(ows, ows_bytes);
+  int32_t* cursor = cv.take<int32_t>((size_t)k + 1);
+  int32_t* cnt = cv.take<int32_t>((size_t)k);  // this chunk's counts
+  const int64_t rows = std::min<int64_t>(n, fit);
+  int32_t* order = cv.take<int32_t>((size_t)rows);
+  FGPU_CHECK(cv.ok(), FGPU_ERR_WORKSPACE, "kmeans_update: workspace too small");
+  const size_t lds = (size_t)k * sizeof(int32_t);
+  for (const void* f : {(const void*)order_count_kernel, (const void*)order_scatter_kernel})
+    FGPU_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const int nv = (dim + 63) / 64;
+  for (int64_t b = 0; b < n; b += rows) {
+    const int64_t nb = std::min<int64_t>(rows, n - b);
+    const unsigned g = (unsigned)((nb + kOrdThreads * kOrdPer - 1) / (kOrdThreads * kOrdPer));
+    int32_t* cc = n <= rows ? counts : cnt;
+    if (cc == cnt) FGPU_TRY(launch1d(fill_i32_kernel, (int64_t)k, 256, s, cnt, (int64_t)k));
+    hipLaunchKernelGGL(order_count_kernel, dim3(g), dim3(kOrdThreads), lds, s, assign + b, nb, k, cc);
+    hipLaunchKernelGGL(exclusive_scan_kernel, dim3(1), dim3(1024), 0, s, cc, k, cursor);
+    hipLaunchKernelGGL(order_scatter_kernel, dim3(g), dim3(kOrdThreads), lds, s, assign + b, nb, k, cursor, order);
+    const dim3 sg((unsigned)((nb + 4 * kOrdSeg - 1) / (4 * kOrdSeg)));
+    const float* xb = x + b * dim;
+    const int32_t* tot = cursor + k;  // the scan's total; the scatter leaves it alone
+#define FGPU_OS(V) \
+  if (nv == V)     \
+    hipLaunchKernelGGL(order_sum_kernel<V>, sg, dim3(256), 0, s, xb, tot, assign + b, order, dim, shift, sums)
+    FGPU_OS(1);
+    FGPU_OS(2);
+    FGPU_OS(3);
+    FGPU_OS(4);
+#undef FGPU_OS
+    if (cc == cnt) FGPU_TRY(launch1d(add_i32_kernel, (int64_t)k, 256, s, counts, cnt, (int64_t)k));
+  }
+  FGPU_HIP(hipGetLastError());
+  return FGPU_OK;
 }
 
 fgpu_status launch_kmeans_finalize(const unsigned long long* sums, const int32_t* counts, int k, int dim, int shift,

@@ -1250,7 +1250,8 @@ int fgpu_fixed_shift(float maxabs, int64_t n) {
 }
 
 size_t fgpu_kmeans_workspace_bytes(int k, int dim) {
-  return carve_bytes<unsigned long long>((size_t)k * dim) + carve_bytes<int32_t>(k);
+  return carve_bytes<unsigned long long>((size_t)k * dim) + carve_bytes<int32_t>(k) +
+         kmeans_order_bytes(k, kOrderedChunk);
 }
 
 fgpu_status fgpu_kmeans_update(const float* dx, int64_t n, const int32_t* d_assign, int k, int dim, int shift,
@@ -1263,7 +1264,10 @@ fgpu_status fgpu_kmeans_update(const float* dx, int64_t n, const int32_t* d_assi
   int32_t* cnt = cv.take<int32_t>(k);
   FGPU_CHECK(cv.ok(), FGPU_ERR_WORKSPACE, "kmeans_update: workspace too small");
   if (d_counts) cnt = d_counts;
-  FGPU_TRY(launch_kmeans_accumulate(dx, n, d_assign, k, dim, shift, sums, cnt, s));
+  // what is left of the workspace groups the rows by centre (a smaller one
+  // than fgpu_kmeans_workspace_bytes, down to the sums and counts, does without)
+  FGPU_TRY(launch_kmeans_accumulate(dx, n, d_assign, k, dim, shift, sums, cnt, cv.base + cv.used,
+                                    ws_bytes - cv.used, s));
   return launch_kmeans_finalize(sums, cnt, k, dim, shift, empty_rule, d_cent, s);
 }
 

@@ -393,9 +393,18 @@ fgpu_status launch_row_gather(const void* d, int64_t nrows, int row_bytes, const
 fgpu_status launch_probe_counts(const uint32_t* probes, int nq, int nprobe, int nlist, const int32_t* offsets,
                                 int32_t* counts, int32_t* offs, hipStream_t s);
 fgpu_status launch_maxabs(const float* x, int64_t count, float* out, hipStream_t s);
+// sums and counts of the rows of each centre; ows (may be null): scratch of
+// kmeans_order_bytes(k, rows), with which kOrderedMinRows rows or more are
+// grouped by centre first, up to `rows` at a time.  Below that the one-atomic-a-
+// coordinate form is as fast; above kOrderedMaxCentres the histogram does not
+// fit LDS.
+constexpr int64_t kOrderedMinRows = 32768;
+constexpr int kOrderedMaxCentres = 16384;
+constexpr int64_t kOrderedChunk = 1 << 20;
+size_t kmeans_order_bytes(int k, int64_t rows);
 fgpu_status launch_kmeans_accumulate(const float* x, int64_t n, const int32_t* assign, int k,
                                      int dim, int shift, unsigned long long* sums, int32_t* counts,
-                                     hipStream_t s);
+                                     void* ows, size_t ows_bytes, hipStream_t s);
 fgpu_status launch_kmeans_finalize(const unsigned long long* sums, const int32_t* counts, int k,
                                    int dim, int shift, int empty_rule, float* cent, hipStream_t s);
 fgpu_status launch_gather_rows(const float* x, int dim, const int32_t* rows, int nrows, float* out,

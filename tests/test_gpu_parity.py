@@ -357,6 +357,38 @@ def test_kmeans_update_bit_exact():
         assert np.array_equal(_bits(_host(c)), _bits(want))
 
 
+@pytest.mark.parametrize("n,k,dim,chunk", [(32768, 1, 128, 0), (32768, 4096, 128, 0), (40001, 300, 96, 0),
+                                           (70000, 1000, 100, 33000), (33000, 16384, 36, 0), (33000, 16385, 36, 0),
+                                           (66001, 7, 200, 40000), (33000, 50, 4, 0)])
+def test_kmeans_update_grouped_rows(n, k, dim, chunk):
+    """From 32768 rows on the rows are grouped by centre before they are summed: one centre holding every row,
+    centres without rows, dims off the 64-lane step, row counts off the grouping and summing tiles, chunks smaller
+    than the rows (a workspace that groups `chunk` rows at a time), the largest centre count and one above it."""
+    _say(f"kmeans_update grouped n={n} k={k} dim={dim} chunk={chunk}")
+    rng = np.random.default_rng(n + k + dim)
+    x = (rng.standard_normal((n, dim)) * 3).astype(np.float32)
+    a = rng.integers(0, k, n).astype(np.int32)
+    if k > 6:
+        a[a == 5] = 3
+    a[: n // 3] = k // 2
+    shift = fg.fixed_shift(float(np.abs(x).max()), n)
+    old = rng.standard_normal((k, dim)).astype(np.float32)
+    c = torch.from_numpy(old.copy()).cuda()
+    dx, da = torch.from_numpy(x).cuda(), torch.from_numpy(a).cuda()
+    if chunk:
+        full = fg.lib.fgpu_kmeans_workspace_bytes(k, dim)
+        ws = torch.empty(full - 4 * ((1 << 20) - chunk), dtype=torch.uint8, device="cuda")
+        cnt = torch.empty(k, dtype=torch.int32, device="cuda")
+        st = fg.lib.fgpu_kmeans_update(dx.data_ptr(), n, da.data_ptr(), k, dim, shift, 1, c.data_ptr(), cnt.data_ptr(),
+                                       ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        assert st == 0
+    else:
+        cnt = fg.kmeans_update(dx, da, c, shift, 1)
+    want, wcnt = oracle.kmeans_update(x, a, old, shift, 1)
+    assert np.array_equal(_host(cnt), wcnt)
+    assert np.array_equal(_bits(_host(c)), _bits(want))
+
+
 @pytest.mark.parametrize("init_mode", [0, 1])
 def test_kmeans_fit_bit_exact(init_mode):
     _say(f"kmeans_fit init={init_mode}")
