@@ -56,18 +56,6 @@ constexpr int kAStage = 4;                  // column tiles (of 32) a stage
 constexpr int kASlots = 32;                 // candidate entries a row (one a column class)
 constexpr uint16_t kAClass = 0x8000u;       // entry: every column of the class
 
-// n2 < 2^norm_exp(n2), the least such power.
-__device__ __forceinline__ int norm_exp(float n2) {
-  int e = 0;
-  (void)frexpf(n2, &e);
-  return e;
-}
-// sc: sqrt(cn_max) 2^sc <= 64.
-__device__ __forceinline__ int column_scale(float cn_max) {
-  const int s = 6 - ((norm_exp(cn_max) + 1) >> 1);
-  return s > 100 ? 100 : s < -100 ? -100 : s;
-}
-
 // Column tiles in MFMA operand order: tile t, fragment c < D / 16: lane (li, h)
 // holds dims 16 c + 8 h .. + 7 of column 32 t + li; the last fragment is the
 // extra block (h = 0: P's three parts, 0 or 65504 past the end, three ones).

@@ -1078,8 +1078,10 @@ int64_t knn_rows(int nq) {
 extern "C" {
 
 size_t fgpu_knn_exact_workspace_bytes(int nq, int64_t n) {
-  return carve_bytes<float>((size_t)std::max(nq, 1)) + carve_bytes<float>((size_t)std::max<int64_t>(n, 1)) +
-         carve_bytes<float>(64) + carve_bytes<float>((size_t)knn_rows(std::max(nq, 1)) * kKnnChunk);
+  const size_t chunked = carve_bytes<float>((size_t)std::max(nq, 1)) +
+                         carve_bytes<float>((size_t)std::max<int64_t>(n, 1)) + carve_bytes<float>(64) +
+                         carve_bytes<float>((size_t)knn_rows(std::max(nq, 1)) * kKnnChunk);
+  return n < kKnnScreenMinRows ? chunked : std::max(chunked, knn_screen_ws_bytes(std::max(nq, 1), n) + 256);
 }
 
 fgpu_status fgpu_knn_exact(const float* dq, int nq, const float* d_base, int64_t n, int dim, int k, int32_t* d_ids,
@@ -1091,6 +1093,8 @@ fgpu_status fgpu_knn_exact(const float* dq, int nq, const float* d_base, int64_t
              "knn_exact: dim must be a multiple of 4 in [4, 256]");
   if (nq == 0) return FGPU_OK;
   hipStream_t s = as_stream(stream);
+  if (((uintptr_t)ws & 15) == 0 && knn_screen_takes(dq, nq, d_base, n, dim, ws_bytes))
+    return launch_knn_screen(dq, nq, d_base, n, dim, k, ws, ws_bytes, d_ids, d_dists, s);
   Carve cv(ws, ws_bytes);
   float* qn = cv.take<float>(nq);
   float* bn = cv.take<float>(n);

@@ -1,5 +1,5 @@
 // fp16_bounds.hpp -- fp16 operands with a stated rounding, for the kernels that
-// bound distances on v_mfma_f32_32x32x16_f16 (screen.hip, assign.hip).
+// bound distances on v_mfma_f32_32x32x16_f16 (screen.hip, assign.hip, knn.hip).
 #pragma once
 
 #include <cmath>
@@ -83,5 +83,18 @@ __device__ __forceinline__ void split3(double v, uint16_t& b1, uint16_t& b2, uin
   b3 = UP ? h_up(r2) : h_down(r2);
 }
 __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) { return (uint32_t)lo | ((uint32_t)hi << 16); }
+
+// ---- scales of rows and columns (assign.hip, knn.hip) -----------------------------
+// n2 < 2^norm_exp(n2), the least such power.
+__device__ __forceinline__ int norm_exp(float n2) {
+  int e = 0;
+  (void)frexpf(n2, &e);
+  return e;
+}
+// sc: sqrt(cn_max) 2^sc <= 64.
+__device__ __forceinline__ int column_scale(float cn_max) {
+  const int s = 6 - ((norm_exp(cn_max) + 1) >> 1);
+  return s > 100 ? 100 : s < -100 ? -100 : s;
+}
 
 }  // namespace fgpu

@@ -54,6 +54,15 @@ constexpr int64_t kAssignMinRows = 32768;
 bool assign_takes(const float* x, int64_t n, const float* c, int nc, int dim, size_t ws_bytes);
 fgpu_status launch_assign(const float* x, int64_t n, const float* c, int nc, int dim, const float* cn_max, void* ws,
                           size_t ws_bytes, int32_t* ids, float* d, hipStream_t s);
+// Exact kNN (k <= 128) of the whole base on fp16 MFMA bounds (knn.hip), without
+// an estimate matrix.  knn_screen_takes: whether it applies (dim 32, 64, 96 or
+// 128, 16-byte aligned arrays, at least kKnnScreenMinRows base rows, a workspace
+// of about knn_screen_ws_bytes) rather than launch_gemm_est + launch_knn_chunk.
+constexpr int64_t kKnnScreenMinRows = 16384;
+size_t knn_screen_ws_bytes(int nq, int64_t n);
+bool knn_screen_takes(const float* x, int nq, const float* c, int64_t n, int dim, size_t ws_bytes);
+fgpu_status launch_knn_screen(const float* x, int nq, const float* c, int64_t n, int dim, int k, void* ws,
+                              size_t ws_bytes, int32_t* ids, float* d, hipStream_t s);
 // Exact kNN over one chunk of <= 4096 base rows c (ids id_base + col), merged
 // into the running top-k in ids/d (k <= 128) when accum != 0.
 fgpu_status launch_knn_chunk(const float* est, int64_t ld, int64_t nrows, int ncols, const float* x, const float* c,

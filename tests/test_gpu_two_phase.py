@@ -410,6 +410,77 @@ def test_knn_exact_bit_exact(k, n, dim):
         assert np.all(gid[:, n:] == -1)
 
 
+def _knn_both(q, x, k):
+    """knn_exact on the workspace it asks for and on one that holds only the chunked form's estimate tile."""
+    dq, dx = torch.from_numpy(q).cuda(), torch.from_numpy(x).cuda()
+    gid, gd = fg.knn_exact(dq, dx, k)
+    r256 = lambda b: -(-b // 256) * 256  # noqa: E731
+    small = r256(4 * len(q)) + r256(4 * len(x)) + 256 + 64 * 4096 * 4
+    cid, cd = fg.knn_exact(dq, dx, k, workspace=torch.empty(small, dtype=torch.uint8, device="cuda"))
+    gid, gd, cid, cd = _host(gid), _host(gd), _host(cid), _host(cd)
+    assert np.array_equal(gid, cid) and np.array_equal(_bits(gd), _bits(cd))
+    return gid, gd
+
+
+@pytest.mark.parametrize("nq,n,dim,k", [(70, 16384, 128, 10), (513, 16417, 96, 100), (1, 40000, 128, 128),
+                                        (33, 100003, 64, 64), (600, 50000, 32, 65), (64, 70001, 128, 1)])
+def test_knn_exact_large_base(nq, n, dim, k):
+    """From 16384 base rows on the base goes through the MFMA bounds once, without estimates: row and query counts
+    off the tiles and workgroups, k at its list edges, rows in cluster order (a query's neighbours are all late),
+    duplicate rows; equal to the chunked form bit for bit, and to the oracle on a sample."""
+    _say(f"knn_exact large base nq={nq} n={n} dim={dim} k={k}")
+    rng = np.random.default_rng(nq + n + dim + k)
+    x = fg.gen_gmm(n, dim, 64, seed=3, sig_lo=0.05, sig_hi=0.2)
+    x = x[np.argsort(x[:, 0], kind="stable")]
+    x[5000:5200] = x[100:300]
+    q = fg.gen_gmm(nq, dim, 64, seed=3, set=1, sig_lo=0.05, sig_hi=0.2)
+    q[nq // 2] = x[150]
+    gid, gd = _knn_both(q, x, k)
+    m = min(nq, 40)
+    oid, od = oracle.knn_exact(q[:m], x, k)
+    assert np.array_equal(gid[:m], oid) and np.array_equal(_bits(gd[:m]), _bits(od))
+
+
+@pytest.mark.parametrize("case", ["ties", "offset", "tiny", "outlier", "nonfinite", "few"])
+def test_knn_exact_large_base_hand_over(case):
+    """Queries the bounds cannot settle take every exact distance: more tied rows than a list holds, a margin as wide
+    as the distances (a large common offset; one row far larger than the rest), queries out of the scales, NaN and
+    infinite rows and queries, fewer finite rows than k.  From one such query to all of them."""
+    _say(f"knn_exact hand-over {case}")
+    rng = np.random.default_rng(len(case))
+    n, nq, dim, k = 20000, 300, 128, 100
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    q = rng.standard_normal((nq, dim)).astype(np.float32)
+    if case == "ties":
+        x[::4] = x[1]
+        q[:17] = x[1]
+        q[17:20] += x[1]
+    elif case == "offset":
+        off = rng.standard_normal(dim).astype(np.float32) * np.float32(1e3)
+        x, q = x + off, q + off
+    elif case == "tiny":
+        x, q = x * np.float32(1e-14), q * np.float32(1e-14)
+        q[3] = 0
+        q[4] *= np.float32(1e8)
+    elif case == "outlier":
+        x[777] *= np.float32(3e4)
+        q[5] *= np.float32(1e6)
+    elif case == "nonfinite":
+        x[50], x[51, 7] = np.nan, np.nan
+        q[2, 3], q[9], q[10, 0] = np.nan, np.inf, -np.inf
+    else:
+        x[60:] = np.nan
+    if case == "few":  # the finite rows, then padding
+        gid = _host(fg.knn_exact(torch.from_numpy(q).cuda(), torch.from_numpy(x).cuda(), k)[0])
+        oid, _ = oracle.knn_exact(q[:24], x[:60], k)
+        assert np.array_equal(gid[:24], oid)
+        return
+    gid, gd = _knn_both(q, x, k)
+    if case != "nonfinite":
+        oid, od = oracle.knn_exact(q[:24], x, k)
+        assert np.array_equal(gid[:24], oid) and np.array_equal(_bits(gd[:24]), _bits(od))
+
+
 def test_reference_default_rerank_m_end_to_end():
     """The reference's default rerank_m = 10000 (defs.h:18) through the
     two-phase scan and the exact rerank, against the oracle."""
