@@ -210,7 +210,7 @@ struct ScreenArgs {
                             // exponent, chunks its list's round-1 work items), (-1, -1), or (-2, 0)
   uint32_t* gminbuf;        // [nq][kMaxChunks][64] round 1: per query, first-list chunk and group, min U bits
   float* thr;               // [nq] T(q)
-  uint2* cand;              // [nq][cand_cap] (vector position, list)
+  uint2* cand;              // [nq][cand_cap] (vector position, list and how far its bound lies below T)
   int cand_cap;
   int* flist;               // [nq] queries handed to the LUT kernel
   int32_t* out_ids;         // [nq][k]

@@ -352,3 +352,28 @@ def test_screen_handed_queries_split_their_probes(dim, m, k, nq, nprobe):
     if nprobe > 1:
         assert st["queries_to_lut_kernel"] >= (nq + 1) // 2
     idx.close()
+
+
+@pytest.mark.parametrize("k,tied", [(1, True), (10, True), (64, True), (10, False), (33, False)])
+def test_screen_rescore_batches(k, tied):
+    """Candidate counts at the 64-candidate batches: every vector of the near list passes the bounds (one code for all:
+    ties by id; or codes a few steps apart), so a query has as many candidates as its list has vectors."""
+    _say(f"rescore batches k={k} tied={tied}")
+    rng = np.random.default_rng(7 * k + tied)
+    dim, m = 128, 32
+    lens = np.array([64, 65, 127, 128, 129, 192, 193, 511, 512])
+    offs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n = int(offs[-1])
+    ids = rng.permutation(n).astype(np.int32)
+    cent = rng.uniform(-1, 1, (lens.size, dim)).astype(np.float32)
+    cb = (rng.standard_normal((m, 256, dim // m)) * 0.02).astype(np.float32)
+    if not tied:
+        cb[:, 1:] = cb[:, :1] + (rng.standard_normal((m, 255, dim // m)) * 1e-3).astype(np.float32)
+    codes = np.zeros((n, m), np.uint8) if tied else rng.integers(0, 256, (n, m), dtype=np.uint8)
+    idx = fg.Index.from_arrays(dim, m, offs, ids, codes, cent, cb)
+    q = np.repeat(cent, 5, axis=0) + (rng.standard_normal((5 * lens.size, dim)) * 0.05).astype(np.float32)
+    st = _check(idx, q.astype(np.float32), cent, cb, offs, ids, codes, 2, k)
+    assert st["queries_with_threshold"] == 5 * lens.size
+    if tied:
+        assert st["max_candidates"] == 512 and st["candidates"] == 5 * n and st["queries_to_lut_kernel"] == 0
+    idx.close()
