@@ -359,24 +359,46 @@ __device__ __forceinline__ void hand_part(const AdcArgs& a, int q, int part, int
   }
 
   uint64_t* mk = reinterpret_cast<uint64_t*>(smem);
-  mk[wave * kWave + lane] = lk;
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll 1
-  for (int w = 1; w < kNW; ++w) wave_merge_sorted64_k(lk, mk[w * kWave + lane]);
+  // The waves' lists to wave 0, pairwise.
+  auto merge_waves = [&]() {
+#pragma unroll
+    for (int half = kNW / 2; half >= 1; half >>= 1) {
+      if (wave >= half && wave < 2 * half) mk[(wave - half) * kWave + lane] = lk;
+      __syncthreads();
+      if (wave < half) wave_merge_sorted64_k(lk, mk[wave * kWave + lane]);
+      __syncthreads();
+    }
+  };
+  merge_waves();
   if (S > 1) {
     uint64_t* parts = a.hand_keys + (size_t)q * a.hand_keys_stride;
-    if (lane < k) parts[(size_t)part * k + lane] = lk;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    if (lane == 0) s_last = __hip_atomic_fetch_add(garr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
-    wave_lds_sync();
+    if (wave == 0) {
+      if (lane < k) parts[(size_t)part * k + lane] = lk;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      if (lane == 0) s_last = __hip_atomic_fetch_add(garr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
+    }
+    __syncthreads();
     if (!s_last) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-#pragma unroll 1
-    for (int j = 0; j < S; ++j)
-      if (j != part) wave_merge_sorted64_k(lk, lane < k ? parts[(size_t)j * k + lane] : kPadKey);
+    // Parts wave, wave + 8, ... of each wave, four loads in flight.
+    lk = kPadKey;
+    for (int j = wave; j < S; j += 4 * kNW) {
+      uint64_t pk[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int jj = j + i * kNW;
+        pk[i] = jj < S && lane < k ? parts[(size_t)jj * k + lane] : kPadKey;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (j + i * kNW < S) wave_merge_sorted64_k(lk, pk[i]);
+    }
+    merge_waves();
   }
-  write_topk(lk, q, k, a);
+  if (wave == 0) {
+    write_topk(lk, q, k, a);
+    if (a.hand_thr && lane == k - 1) a.hand_thr[q] = key_dist(lk);
+  }
 }
 
 template <int D, int M>
@@ -386,12 +408,12 @@ __global__ __launch_bounds__(kNT) void adc_hand_kernel(AdcArgs a) {
   __shared__ int s_list[kHandProbes];
   __shared__ float s_lb[kHandProbes];
   __shared__ int s_next, s_last;
-  const int count = min(*a.qcount, a.nq);
+  const int count = a.qlist ? min(*a.qcount, a.nq) : a.nq;
   if (count <= 0) return;
   const int fit = (int)min((long long)a.nprobe, a.hand_keys_stride / a.k);  // parts a query's region holds
   const int S = max(1, min(fit, (int)gridDim.x / count));
   for (long long it = blockIdx.x; it < (long long)count * S; it += gridDim.x) {
-    const int q = a.qlist[it / S];
+    const int q = a.qlist ? a.qlist[it / S] : (int)(it / S);
     if (q >= 0 && q < a.nq)
       hand_part<D, M>(a, q, (int)(it % S), S, smem, s_thr, s_list, s_lb, s_next, s_last);
     __syncthreads();
@@ -986,7 +1008,7 @@ fgpu_status launch_adc_plain(int dim, int m, const AdcArgs& a, hipStream_t s) {
 }
 
 fgpu_status launch_adc_hand(int dim, int m, const AdcArgs& a, hipStream_t s) {
-  FGPU_CHECK(a.k >= 1 && a.k <= 64 && a.qlist && a.qcount && a.hand && a.hand_keys && a.nprobe >= 1 &&
+  FGPU_CHECK(a.k >= 1 && a.k <= 64 && (!a.qlist || a.qcount) && a.hand && a.hand_keys && a.nprobe >= 1 &&
                  a.nprobe <= kHandProbes,
              FGPU_ERR_ARG, "adc: bad query list launch");
   if (a.nq <= 0) return FGPU_OK;

@@ -191,6 +191,16 @@ AdcArgs adc_args(const fgpu_index* ix, const float* dq, int nq, const uint32_t* 
   return a;
 }
 
+// Searches of at most this many queries take the LUT kernel with every query's
+// probes split over the GPU rather than the screen's nine launches or one
+// workgroup a query (but not the flow kernel's: 96 dims in 16 codes, 48 probes,
+// 64 queries 36 against 42 us).  Measured (us, screen / this): 128 dims in 16
+// codes, 100k vectors, 16 probes: 51 / 25 for 1 query, 82 / 36 for 64; 32 codes,
+// 1M, 32 probes: 57 / 30 and 92 / 46; 64 codes, 1M, 128 probes, k 64: 89 / 59
+// and 550 / 70; one workgroup a query, 96 dims in 32 codes, 100 probes: 48 / 37
+// and 62 / 52, 63 / 64 for 128.
+constexpr int kSmallBatch = 64;
+
 // The screen's workspace, carved from `base` (fgpu_search, after the probe
 // arrays).  The counters, per-list counts and per-query candidate counts are
 // one contiguous block that the first screen kernel zeroes.
@@ -456,12 +466,11 @@ size_t fgpu_coarse_workspace_bytes(int nq, int nlist) {
 }  // extern "C"
 
 namespace {
-// fgpu_coarse_search; with side != nullptr its first select launch also
-// stores side_val at *side (the scan's query counter, so the scan needs no
-// reset kernel of its own).
+// fgpu_coarse_search; its first select launch stores the side words (so the
+// scan needs no kernel of its own to set them).
 fgpu_status coarse_search(const fgpu_index* ix, const float* dq, int nq, int nprobe, float prune_ratio,
-                          uint32_t* d_ids, float* d_dists, void* ws, size_t ws_bytes, void* stream, int* side,
-                          int side_val, unsigned long long* stats = nullptr) {
+                          uint32_t* d_ids, float* d_dists, void* ws, size_t ws_bytes, void* stream,
+                          const SelectSide& side, unsigned long long* stats = nullptr) {
   // An empty batch may come with empty (null) arrays.
   FGPU_CHECK(ix && ws && (nq == 0 || (dq && d_ids && d_dists)), FGPU_ERR_ARG, "coarse_search: null argument");
   FGPU_CHECK(((uintptr_t)ws & 15) == 0, FGPU_ERR_ARG, "coarse_search: workspace must be 16-byte aligned");
@@ -484,7 +493,7 @@ fgpu_status coarse_search(const fgpu_index* ix, const float* dq, int nq, int npr
     FGPU_TRY(launch_select_exact(est, ld, nb, ix->nlist, dq + b0 * ix->dim, ix->d_centroids, ix->dim,
                                  ix->d_cnorm_max, nprobe, 1, prune_ratio,
                                  reinterpret_cast<int32_t*>(d_ids) + b0 * nprobe, d_dists + b0 * nprobe, s,
-                                 b0 == 0 ? side : nullptr, side_val, stats));
+                                 b0 == 0 ? side : SelectSide{}, stats));
   }
   return FGPU_OK;
 }
@@ -494,14 +503,14 @@ extern "C" {
 
 fgpu_status fgpu_coarse_search(const fgpu_index* ix, const float* dq, int nq, int nprobe, float prune_ratio,
                                uint32_t* d_ids, float* d_dists, void* ws, size_t ws_bytes, void* stream) {
-  return coarse_search(ix, dq, nq, nprobe, prune_ratio, d_ids, d_dists, ws, ws_bytes, stream, nullptr, 0);
+  return coarse_search(ix, dq, nq, nprobe, prune_ratio, d_ids, d_dists, ws, ws_bytes, stream, {});
 }
 
 fgpu_status fgpu_coarse_search_stats(const fgpu_index* ix, const float* dq, int nq, int nprobe, float prune_ratio,
                                      uint32_t* d_ids, float* d_dists, unsigned long long* d_stats, void* ws,
                                      size_t ws_bytes, void* stream) {
   FGPU_CHECK(d_stats, FGPU_ERR_ARG, "coarse_search_stats: null stats");
-  return coarse_search(ix, dq, nq, nprobe, prune_ratio, d_ids, d_dists, ws, ws_bytes, stream, nullptr, 0, d_stats);
+  return coarse_search(ix, dq, nq, nprobe, prune_ratio, d_ids, d_dists, ws, ws_bytes, stream, {}, d_stats);
 }
 
 fgpu_status fgpu_prune_probes(uint32_t* d_probe_ids, const float* d_probe_dists, int nq, int nprobe, float prune_ratio,
@@ -612,8 +621,10 @@ size_t fgpu_search_workspace_bytes(int nq, int nlist, int nprobe) {
   // The coarse step's estimate tile and the screen's buffers are never live
   // at once, so they share one region (no screen beyond kScreenMaxLists lists).
   const size_t screen = nlist <= kScreenMaxLists ? ScreenWs::bytes(nq, nlist, nprobe) : 0;
+  const size_t coarse = fgpu_coarse_workspace_bytes(nq, nlist);
+  // (A small batch's select sets up the scan's words while it reads the tile.)
   return carve_bytes<uint32_t>((size_t)nq * nprobe) + carve_bytes<float>((size_t)nq * nprobe) +
-         carve_bytes<int>(1) + std::max(fgpu_coarse_workspace_bytes(nq, nlist), screen);
+         carve_bytes<int>(1) + (nq <= kSmallBatch ? coarse + screen : std::max(coarse, screen));
 }
 
 fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprobe, int k, float prune_ratio,
@@ -637,10 +648,41 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   auto mark = [&](int i) { return ev ? hipEventRecord(ev[i], s) : hipSuccess; };
   FGPU_HIP(mark(0));
   ScreenWs sw;
+  // A small batch: coarse, then the LUT kernel with split probes
+  // (launch_adc_hand) in the screen's buffers, beside the coarse step's tile.
+  const size_t sbytes = nq <= kSmallBatch ? ScreenWs::bytes(nq, ix->nlist, nprobe) : 0;
+  if (nq > 0 && nq <= kSmallBatch && ix->opt_screen && ix->opt_list_skip && k <= 64 && nprobe >= 1 && nprobe <= 256 &&
+      (ix->screen_ok || flow_grid(ix->dim, ix->m, nq, nprobe) == 0) && ix->nlist <= kScreenMaxLists &&
+      ((uintptr_t)ix->d_codebook & 15) == 0 && rest_bytes > sbytes &&
+      rest_bytes - sbytes >= fgpu_coarse_workspace_bytes(nq, ix->nlist) &&
+      sw.carve(rest, rest_bytes, nq, ix->nlist, nprobe)) {
+    ScreenArgs sa{};
+    sa.nprobe = nprobe;
+    sa.ctr = sw.zero;
+    sa.gminbuf = sw.gminbuf;
+    sa.arec = sw.arec;
+    AdcArgs a = adc_args(ix, dq, nq, pid, pd, nprobe, k, d_out_ids, d_out_dists);
+    screen_hand(sa, &a);
+    a.qlist = nullptr;
+    a.hand_thr = sw.thr;
+    SelectSide side;
+    side.zero = sw.zero;
+    side.nzero = (int)ScreenWs::zero_words(nq, ix->nlist);
+    side.flag_at = kCtrFlag;
+    side.flag = nq;
+    side.hand = a.hand;
+    side.hand_stride = a.hand_stride;
+    FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, static_cast<char*>(rest) + sbytes,
+                           rest_bytes - sbytes, stream, side));
+    for (int i = 1; i < kStageEvents - 1; ++i) FGPU_HIP(mark(i));  // no screen stages
+    FGPU_TRY(launch_adc_hand(ix->dim, ix->m, a, s));
+    FGPU_HIP(mark(kStageEvents - 1));
+    return FGPU_OK;
+  }
   if (ix->screen_ok && ix->opt_screen && k <= 64 && nq > 0 && ((uintptr_t)dq & 15) == 0 &&
       ix->nlist <= kScreenMaxLists && (int64_t)nq * nprobe < INT32_MAX &&
       sw.carve(rest, rest_bytes, nq, ix->nlist, nprobe)) {
-    FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream, nullptr, 0));
+    FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream, {}));
     FGPU_HIP(mark(1));
     ScreenArgs sa{dq, ix->d_centroids, ix->d_offsets, ix->d_codes, ix->d_ids, ix->d_codebook, ix->d_cb16,
                   ix->d_vext, ix->d_rmax, pid, pd, nq, nprobe, k, ix->nlist};
@@ -671,8 +713,10 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   // The scan claims queries from a counter that starts at its grid size; the
   // coarse step's select stores that value on the way.
   const int grid = flow_grid(ix->dim, ix->m, nq, nprobe);
-  FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream,
-                         grid > 0 ? qctr : nullptr, grid));
+  SelectSide side;
+  side.ctr = grid > 0 ? qctr : nullptr;
+  side.ctr_val = grid;
+  FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream, side));
   for (int i = 1; i < kStageEvents - 1; ++i) FGPU_HIP(mark(i));  // no screen stages
   AdcArgs a = adc_args(ix, dq, nq, pid, pd, nprobe, k, d_out_ids, d_out_dists);
   a.qctr = qctr;

@@ -637,6 +637,20 @@ __device__ __forceinline__ void select_row(const float (&val)[VPL], int64_t row,
   }
 }
 
+// The launch's side words, by its first workgroup.
+__device__ __forceinline__ void side_words(const SelectSide& s, int64_t nrows) {
+  if (blockIdx.x != 0) return;
+  if (s.ctr && threadIdx.x == 0) *s.ctr = s.ctr_val;
+  if (s.zero)
+    for (int i = threadIdx.x; i < s.nzero; i += blockDim.x) s.zero[i] = i == s.flag_at ? s.flag : 0;
+  if (s.hand)
+    for (int64_t r = threadIdx.x; r < nrows; r += blockDim.x) {
+      uint32_t* h = s.hand + r * s.hand_stride;
+      *reinterpret_cast<uint64_t*>(h) = kPadKey;
+      h[2] = 0u;
+    }
+}
+
 // One wave per row over the estimate matrix est (row stride ld).  The
 // estimates may leave out the row's own norm (a shift of the whole row: the
 // p-th estimate and the candidate set move with it); the margin takes the
@@ -647,14 +661,14 @@ __global__ __launch_bounds__(256) void select_exact_kernel(
     const E* __restrict__ est, int64_t ld, int64_t nrows, int ncols,
     const float* __restrict__ x, const float* __restrict__ c, int dim,
     const float* __restrict__ cn_max, float kappa, int p, int prune,
-    float prune_ratio, int32_t* __restrict__ out_ids, float* __restrict__ out_d, int* side, int side_val,
+    float prune_ratio, int32_t* __restrict__ out_ids, float* __restrict__ out_d, SelectSide side,
     const uint8_t* __restrict__ rsh, unsigned long long* __restrict__ stats) {
   __shared__ uint32_t hist_s[4][256];
   __shared__ int cand_s[4][kCandCap];
   __shared__ __align__(16) float x_s[4][256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
-  if (side && blockIdx.x == 0 && threadIdx.x == 0) *side = side_val;  // the caller's one-word side write
+  side_words(side, nrows);
   if (row >= nrows) return;  // whole wave leaves; no workgroup barrier follows
   float* xs = x_s[wave];
   float xnr = 0.0f;
@@ -722,7 +736,7 @@ __global__ __launch_bounds__(256) void select_min_kernel(
     const E* __restrict__ est, int64_t ld, int64_t nrows, int ncols,
     const float* __restrict__ x, const float* __restrict__ c, int dim,
     const float* __restrict__ cn_max, float kappa, int prune, float prune_ratio,
-    int32_t* __restrict__ out_ids, float* __restrict__ out_d, int* side, int side_val,
+    int32_t* __restrict__ out_ids, float* __restrict__ out_d, SelectSide side,
     const uint8_t* __restrict__ rsh, unsigned long long* __restrict__ stats) {
   __shared__ int cand_s[4][kCandCap];
   __shared__ __align__(16) float x_s[4][256];
@@ -731,7 +745,7 @@ __global__ __launch_bounds__(256) void select_min_kernel(
   constexpr int PIECE = V * kWave;     // columns a piece
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
-  if (side && blockIdx.x == 0 && threadIdx.x == 0) *side = side_val;  // the caller's one-word side write
+  side_words(side, nrows);
   if (row >= nrows) return;  // whole wave leaves; no workgroup barrier follows
   float* xs = x_s[wave];
   int* cand = cand_s[wave];
@@ -937,17 +951,17 @@ fgpu_status launch_knn_t(const float* est, int64_t ld, int64_t nrows, int ncols,
 template <int VPL>
 fgpu_status launch_select_t(const void* est, int64_t ld, int64_t nrows, int ncols, const float* x,
                             const float* c, int dim, const float* cn_max, float kappa,
-                            int p, int prune, float prune_ratio, int32_t* ids, float* d, int* side, int side_val,
+                            int p, int prune, float prune_ratio, int32_t* ids, float* d, const SelectSide& side,
                             hipStream_t s, unsigned long long* stats) {
   const int64_t blocks = (nrows + 3) / 4;
   if constexpr (kEstHalf)
     hipLaunchKernelGGL((select_exact_kernel<VPL, uint16_t>), dim3((unsigned)blocks), dim3(256), 0, s,
                        static_cast<const uint16_t*>(est), ld, nrows, ncols, x, c, dim, cn_max, kappa, p, prune,
-                       prune_ratio, ids, d, side, side_val, est_row_shift(const_cast<void*>(est), nrows, ld), stats);
+                       prune_ratio, ids, d, side, est_row_shift(const_cast<void*>(est), nrows, ld), stats);
   else
     hipLaunchKernelGGL((select_exact_kernel<VPL, float>), dim3((unsigned)blocks), dim3(256), 0, s,
                        static_cast<const float*>(est), ld, nrows, ncols, x, c, dim, cn_max, kappa, p, prune,
-                       prune_ratio, ids, d, side, side_val, nullptr, stats);
+                       prune_ratio, ids, d, side, nullptr, stats);
   FGPU_HIP(hipGetLastError());
   return FGPU_OK;
 }
@@ -1017,8 +1031,8 @@ static float coarse_kappa(int dim) {
 
 fgpu_status launch_select_exact(const void* est, int64_t ld, int64_t nrows, int ncols, const float* x,
                                 const float* c, int dim, const float* cn_max, int p,
-                                int prune, float prune_ratio, int32_t* ids, float* d, hipStream_t s, int* side,
-                                int side_val, unsigned long long* stats) {
+                                int prune, float prune_ratio, int32_t* ids, float* d, hipStream_t s,
+                                const SelectSide& side, unsigned long long* stats) {
   FGPU_CHECK(ld % 8 == 0, FGPU_ERR_ARG, "select: row stride must be a multiple of 8");
   FGPU_CHECK(p >= 1 && p <= kSelectMax && p <= ncols, FGPU_ERR_UNSUPPORTED, "select: need 1 <= p <= min(256, ncols)");
   FGPU_CHECK(dim <= 256, FGPU_ERR_UNSUPPORTED, "select: dim must be <= 256");
@@ -1028,19 +1042,18 @@ fgpu_status launch_select_exact(const void* est, int64_t ld, int64_t nrows, int 
     const dim3 grid((unsigned)((nrows + 3) / 4));
     if constexpr (kEstHalf)
       hipLaunchKernelGGL(select_min_kernel<uint16_t>, grid, dim3(256), 0, s, static_cast<const uint16_t*>(est), ld,
-                         nrows, ncols, x, c, dim, cn_max, kappa, prune, prune_ratio, ids, d, side, side_val,
+                         nrows, ncols, x, c, dim, cn_max, kappa, prune, prune_ratio, ids, d, side,
                          est_row_shift(const_cast<void*>(est), nrows, ld), stats);
     else
       hipLaunchKernelGGL(select_min_kernel<float>, grid, dim3(256), 0, s, static_cast<const float*>(est), ld, nrows,
-                         ncols, x, c, dim, cn_max, kappa, prune, prune_ratio, ids, d, side, side_val, nullptr,
-                         stats);
+                         ncols, x, c, dim, cn_max, kappa, prune, prune_ratio, ids, d, side, nullptr, stats);
     FGPU_HIP(hipGetLastError());
     return FGPU_OK;
   }
 #define FGPU_SEL(V) \
   if (ncols <= (V) * kWave) \
     return launch_select_t<V>(est, ld, nrows, ncols, x, c, dim, cn_max, kappa, p, prune, prune_ratio, ids, d, side, \
-                              side_val, s, stats)
+                              s, stats)
   FGPU_SEL(1);
   FGPU_SEL(2);
   FGPU_SEL(4);

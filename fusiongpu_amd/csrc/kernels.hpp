@@ -27,18 +27,28 @@ fgpu_status launch_gemm_est(const float* x, int64_t nrows, const float* c, int n
 fgpu_status launch_gemm_est_sel(const float* x, int64_t nrows, const float* c, int ncols, int dim, const float* cn,
                                 const float* cn_max, void* est, int64_t ld, hipStream_t s);
 int64_t est_sel_ld(int ncols);
+// Words the coarse select stores for the kernels after it: *ctr = ctr_val (the
+// flow scan's query counter); zero[0 .. nzero) = 0 except zero[flag_at] = flag;
+// each row's hand[row stride .. + 2] = kPadKey and 0 (AdcArgs::hand).
+struct SelectSide {
+  int* ctr = nullptr;
+  int ctr_val = 0;
+  int* zero = nullptr;
+  int nzero = 0, flag_at = 0, flag = 0;
+  uint32_t* hand = nullptr;
+  long long hand_stride = 0;
+};
 // Per row: the p nearest columns by exact device-form L2, chosen from the
 // estimates of launch_gemm_est_sel with a rigorous error margin.  ids
 // are int32 bit patterns; with prune != 0 a column farther than
-// best*prune_ratio gets 0xFFFFFFFF.  With side != nullptr the launch also
-// stores side_val at *side (one word, for the next kernel on the stream).
+// best*prune_ratio gets 0xFFFFFFFF.  side: words stored on the way.
 // stats (nullptr = off): adds the columns re-scored exactly to stats[0] and
 // the rows that re-scored every column to stats[1].
 fgpu_status launch_select_exact(const void* est, int64_t ld, int64_t nrows, int ncols,
                                 const float* x, const float* c, int dim,
                                 const float* cn_max, int p, int prune, float prune_ratio,
-                                int32_t* out_ids, float* out_d, hipStream_t s, int* side = nullptr,
-                                int side_val = 0, unsigned long long* stats = nullptr);
+                                int32_t* out_ids, float* out_d, hipStream_t s, const SelectSide& side = {},
+                                unsigned long long* stats = nullptr);
 // The nearest column of every row (p = 1) without an estimate matrix
 // (assign.hip): ids and exact distances; ws holds its column tiles and each
 // row's candidates.  assign_takes: whether it applies (dim 32, 64, 96 or 128,
@@ -119,17 +129,19 @@ struct AdcArgs {
   // it equals the grid it launches (flow_grid).
   int qctr_preset = 0;
   // launch_adc_hand only: the queries to search, qlist[0 .. *qcount) (device
-  // memory; the count is read on the device); per query q, hand[q hand_stride]:
-  // a 64-bit key above every member of its top-k (kPadKey: none known) and an
-  // arrival count (0); and room for the parts' keys at
+  // memory; the count is read on the device; nullptr: all nq); per query q,
+  // hand[q hand_stride]: a 64-bit key above every member of its top-k (kPadKey:
+  // none known) and an arrival count (0); and room for the parts' keys at
   // hand_keys[q hand_keys_stride].  The screen's rescore writes the first
-  // three; the keys live where its pair records were.
+  // three (for all nq, the coarse select: SelectSide); the keys live where its
+  // pair records were.  hand_thr (may be null): [nq] each query's k-th distance.
   const int* qlist = nullptr;
   const int* qcount = nullptr;
   uint32_t* hand = nullptr;
   long long hand_stride = 0;
   uint64_t* hand_keys = nullptr;
   long long hand_keys_stride = 0;
+  float* hand_thr = nullptr;
 };
 // Id written to every slot of a query whose result a bounded-wait give-up may
 // have touched (the reference's padding id is -1; it never writes -2).

@@ -371,9 +371,49 @@ def test_screen_rescore_batches(k, tied):
         cb[:, 1:] = cb[:, :1] + (rng.standard_normal((m, 255, dim // m)) * 1e-3).astype(np.float32)
     codes = np.zeros((n, m), np.uint8) if tied else rng.integers(0, 256, (n, m), dtype=np.uint8)
     idx = fg.Index.from_arrays(dim, m, offs, ids, codes, cent, cb)
-    q = np.repeat(cent, 5, axis=0) + (rng.standard_normal((5 * lens.size, dim)) * 0.05).astype(np.float32)
+    q = np.repeat(cent, 8, axis=0) + (rng.standard_normal((8 * lens.size, dim)) * 0.05).astype(np.float32)
     st = _check(idx, q.astype(np.float32), cent, cb, offs, ids, codes, 2, k)
-    assert st["queries_with_threshold"] == 5 * lens.size
+    assert st["queries_with_threshold"] == 8 * lens.size
     if tied:
-        assert st["max_candidates"] == 512 and st["candidates"] == 5 * n and st["queries_to_lut_kernel"] == 0
+        assert st["max_candidates"] == 512 and st["candidates"] == 8 * n and st["queries_to_lut_kernel"] == 0
+    idx.close()
+
+
+@pytest.mark.parametrize("dim,m,nq,nprobe,k", [(128, 16, 1, 1, 1), (128, 32, 64, 9, 10), (128, 64, 5, 37, 64),
+                                               (96, 48, 63, 37, 33), (96, 32, 2, 65, 20), (96, 16, 64, 70, 64),
+                                               (96, 16, 3, 12, 10)])
+def test_small_batches_split_their_probes(dim, m, nq, nprobe, k):
+    """Up to 64 queries: the LUT kernel with every query's probes split over the GPU (the flow kernel for the
+    geometries without a screen up to 64 probes).  One probe, more parts than a query's keys have room for, empty and
+    short lists, pruned probes, a misaligned query array; bit-exact, also replayed from a captured graph."""
+    _say(f"small batch dim={dim} m={m} nq={nq} nprobe={nprobe} k={k}")
+    rng = np.random.default_rng(dim + m + nq + nprobe)
+    lens = rng.integers(0, 400, 80)
+    lens[:6] = [0, 1, k - 1, 127, 129, 1500]
+    offs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n = int(offs[-1])
+    ids = rng.permutation(n).astype(np.int32)
+    codes = rng.integers(0, 256, (n, m), dtype=np.uint8)
+    codes[n // 2:] = codes[: n - n // 2]  # ties across lists
+    cent = (rng.standard_normal((lens.size, dim)) * 0.3).astype(np.float32)
+    cb = (rng.standard_normal((m, 256, dim // m)) * 0.1).astype(np.float32)
+    idx = fg.Index.from_arrays(dim, m, offs, ids, codes, cent, cb)
+    q = (cent[rng.integers(0, 12, nq)] + rng.standard_normal((nq, dim)) * 0.05).astype(np.float32)
+    for prune in (100.0, 1.3):
+        _check(idx, q, cent, cb, offs, ids, codes, nprobe, k, prune_ratio=prune, screened=False)
+    buf = torch.empty(q.size + 1, dtype=torch.float32, device="cuda")
+    dq = buf[1:].view(nq, dim)
+    dq.copy_(torch.from_numpy(q))
+    _check(idx, q, cent, cb, offs, ids, codes, nprobe, k, dq=dq, screened=False)
+    dq = torch.from_numpy(q).cuda()
+    want = [_host(t) for t in idx.search(dq, nprobe, k)]
+    ws = torch.empty(idx.search_workspace_bytes(nq, nprobe), dtype=torch.uint8, device="cuda")
+    out = (torch.empty((nq, k), dtype=torch.int32, device="cuda"), torch.empty((nq, k), device="cuda"))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        idx.search(dq, nprobe, k, workspace=ws, out=out)
+    for _ in range(3):
+        out[0].fill_(-7)
+        g.replay()
+        assert np.array_equal(_host(out[0]), want[0]) and np.array_equal(_bits(_host(out[1])), _bits(want[1]))
     idx.close()
