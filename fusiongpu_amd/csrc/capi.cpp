@@ -151,7 +151,7 @@ fgpu_status finish_index(fgpu_index* ix, hipStream_t s) {
       se = std::max(-60, std::min(60, se));
     }
     ix->screen_scale_exp = se;
-    if (alloc((void**)&ix->d_cb16, (size_t)ix->dim * kPQK * sizeof(uint16_t)) &&
+    if (alloc((void**)&ix->d_cb16, screen_codebook_words(ix->dim, ix->m) * sizeof(uint16_t)) &&
         alloc((void**)&ix->d_vext, sizeof(uint4) * (size_t)std::max<int64_t>(ix->total, 1)) &&
         alloc((void**)&xmax, 256)) {
       FGPU_TRY(launch_screen_prep(ix->d_codebook, ix->m, ix->dim / ix->m, se, ix->d_codes, ix->total, ix->d_cb16,
@@ -193,13 +193,35 @@ AdcArgs adc_args(const fgpu_index* ix, const float* dq, int nq, const uint32_t* 
 
 // Searches of at most this many queries take the LUT kernel with every query's
 // probes split over the GPU rather than the screen's nine launches or one
-// workgroup a query (but not the flow kernel's: 96 dims in 16 codes, 48 probes,
-// 64 queries 36 against 42 us).  Measured (us, screen / this): 128 dims in 16
+// workgroup a query (96 dims in 16 or 32 codes keep the flow kernel: 16 codes,
+// 48 probes, 64 queries 36 against 42 us).  Measured (us, screen / this): 128 dims in 16
 // codes, 100k vectors, 16 probes: 51 / 25 for 1 query, 82 / 36 for 64; 32 codes,
 // 1M, 32 probes: 57 / 30 and 92 / 46; 64 codes, 1M, 128 probes, k 64: 89 / 59
 // and 550 / 70; one workgroup a query, 96 dims in 32 codes, 100 probes: 48 / 37
 // and 62 / 52, 63 / 64 for 128.
 constexpr int kSmallBatch = 64;
+// Whether a search of more than kSmallBatch queries takes the screen (when the
+// index has it) or the LUT kernels.  The screen's cost starts at about 80 us and
+// grows slowly; the flow kernel (flow: it applies) takes a round of one query a CU,
+// 20-30 us where the data's clusters let it skip lists, 60-120 us where they do
+// not, and the screen's threshold is weak for k > 32.  So, us flow / screen:
+//   * up to 256 queries (one round) the flow kernel: 128 dims in 32 codes, 1M,
+//     32 probes, 256 queries: 44 / 96 on C2's clusters, 125 / 173 on one Gaussian
+//     blob (512 queries: 58 / 98 and 211 / 181);
+//   * up to 2048 for k > 32: k 64, 155 / 239 (2048 queries, C2's clusters), k 50
+//     in 16 codes of 96 dims, wide clusters: 559 / 1201;
+//   * codes of 3 or 6 dims (96 in 32 or 16): k <= 32 from 3072 queries on (48
+//     probes, 16 codes, 2000 queries 128 / 126, 4000 223 / 145; 32 codes 129 / 147
+//     and 224 / 170); past 64 probes, where one workgroup scans each query, from
+//     768 (32 codes, 100 probes, 512 queries 103 / 130, 1000 168 / 133).
+// Indexes below kScreenAnyBatch vectors keep the screen at every batch size: its
+// counters (fgpu_search_screen_stats) describe such searches.
+constexpr int kFlowRound = 256, kFlowWideK = 2048, kScreen3Flow = 3072, kScreen3Plain = 768;
+constexpr int64_t kScreenAnyBatch = 65536;
+bool screen_pays(const fgpu_index* ix, int nq, int k, bool flow) {
+  if (ix->dim / ix->m % 3 == 0) return flow ? k <= 32 && nq >= kScreen3Flow : nq >= kScreen3Plain;
+  return !flow || ix->total < kScreenAnyBatch || nq > (k > 32 ? kFlowWideK : kFlowRound);
+}
 
 // The screen's workspace, carved from `base` (fgpu_search, after the probe
 // arrays).  The counters, per-list counts and per-query candidate counts are
@@ -247,7 +269,9 @@ struct ScreenWs {
 // per-list counts and compact bucket offsets, and the screen's workspace.
 // Batches below this many queries keep phase 1 in the two-phase kernel (the
 // screen's fixed launches cost more than they save there).
-constexpr int kTpScreenMinQueries = 1024;
+// Codes of 3 or 6 dims: 2048 (96 dims, us, kernel / screen: 16 codes, 1024
+// queries 127 / 160, 2048 201 / 203, 5000 392 / 355; 64 probes 262 / 271, 481 / 375).
+constexpr int kTpScreenMinQueries = 1024, kTpScreen3MinQueries = 2048;
 constexpr int kTpVqMax = 131072;  // virtual queries a chunk (fuller 32-row MFMA groups per list)
 struct TpScreenWs {
   uint32_t* vprobe = nullptr;
@@ -648,11 +672,12 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   auto mark = [&](int i) { return ev ? hipEventRecord(ev[i], s) : hipSuccess; };
   FGPU_HIP(mark(0));
   ScreenWs sw;
+  const bool flow = flow_grid(ix->dim, ix->m, nq, nprobe) > 0;
   // A small batch: coarse, then the LUT kernel with split probes
   // (launch_adc_hand) in the screen's buffers, beside the coarse step's tile.
   const size_t sbytes = nq <= kSmallBatch ? ScreenWs::bytes(nq, ix->nlist, nprobe) : 0;
   if (nq > 0 && nq <= kSmallBatch && ix->opt_screen && ix->opt_list_skip && k <= 64 && nprobe >= 1 && nprobe <= 256 &&
-      (ix->screen_ok || flow_grid(ix->dim, ix->m, nq, nprobe) == 0) && ix->nlist <= kScreenMaxLists &&
+      (ix->dim / ix->m % 3 != 0 || !flow) && ix->nlist <= kScreenMaxLists &&
       ((uintptr_t)ix->d_codebook & 15) == 0 && rest_bytes > sbytes &&
       rest_bytes - sbytes >= fgpu_coarse_workspace_bytes(nq, ix->nlist) &&
       sw.carve(rest, rest_bytes, nq, ix->nlist, nprobe)) {
@@ -679,7 +704,7 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
     FGPU_HIP(mark(kStageEvents - 1));
     return FGPU_OK;
   }
-  if (ix->screen_ok && ix->opt_screen && k <= 64 && nq > 0 && ((uintptr_t)dq & 15) == 0 &&
+  if (ix->screen_ok && ix->opt_screen && k <= 64 && nq > 0 && screen_pays(ix, nq, k, flow) && ((uintptr_t)dq & 15) == 0 &&
       ix->nlist <= kScreenMaxLists && (int64_t)nq * nprobe < INT32_MAX &&
       sw.carve(rest, rest_bytes, nq, ix->nlist, nprobe)) {
     FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream, {}));
@@ -853,7 +878,8 @@ fgpu_status two_phase(const fgpu_index* ix, const float* dq, int nq, const uint3
   // select.  The virtual queries' buffers take the end of the workspace; the
   // pools and cutoff rows the rest.
   const bool tp_screen = ix->opt_two_phase_screen == 2 ||
-                         (ix->opt_two_phase_screen == 0 && (int64_t)nq >= kTpScreenMinQueries);
+                         (ix->opt_two_phase_screen == 0 &&
+                          nq >= (ix->dim / ix->m % 3 == 0 ? kTpScreen3MinQueries : kTpScreenMinQueries));
   if (tp_screen && ix->screen_ok && ix->opt_screen && limit_k <= 64 && p1 >= 1 && screen_supported(ix->dim, ix->m) &&
       ix->nlist <= kScreenMaxLists && ((uintptr_t)dq & 15) == 0) {
     // With FGPU_OPT_STAGE_EVENTS, the stage events of fgpu_search_stage_times

@@ -183,7 +183,7 @@ struct ScreenArgs {
   const uint8_t* codes;     // [total][m]
   const int32_t* vec_ids;   // [total]
   const float* codebook;    // [m][256][dim/m] fp32
-  const uint16_t* cb16;     // [m][256][dim/m] fp16 of the codebook times 2^scale_exp (nearest, flushed below 2^-14)
+  const uint16_t* cb16;     // [m][256][dim/m, padded] fp16 of the codebook times 2^scale_exp (nearest, flushed below 2^-14)
   const uint4* vext;        // [total] per-vector extra block (screen_prep)
   const float* rmax;        // [nlist]
   const uint32_t* probes;   // [nq][nprobe]; ids >= nlist are skipped
@@ -237,6 +237,8 @@ struct ScreenArgs {
   const hipEvent_t* events = nullptr;
 };
 bool screen_supported(int dim, int m);
+// fp16 values of an index's screen codebook (codewords padded to whole LDS reads).
+size_t screen_codebook_words(int dim, int m);
 // Words of ScreenArgs::gminbuf for nq queries.
 int64_t screen_gmin_words(int nq);
 // The fp16 codebook (times 2^scale_exp) and the per-vector extra blocks of an

@@ -161,11 +161,15 @@ __global__ __launch_bounds__(256) void screen_prep_kernel(const float* __restric
 }
 
 // The codebook times 2^S in fp16 (nearest, flushed below 2^-14), as the
-// screen's B operand.  The scaling is exact in double.
-__global__ __launch_bounds__(256) void cb_f16_kernel(const float* __restrict__ cb, int64_t n, int scale_exp,
-                                                     uint16_t* __restrict__ out) {
+// screen's B operand, each codeword padded with zeros to `pad` values
+// (screen_pad: one aligned LDS read a code).  The scaling is exact in double.
+__global__ __launch_bounds__(256) void cb_f16_kernel(const float* __restrict__ cb, int64_t words, int sub, int pad,
+                                                     int scale_exp, uint16_t* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = h_rn((float)((double)cb[i] * ldexp(1.0, scale_exp)));
+  if (i >= words * pad) return;
+  const int64_t w = i / pad;
+  const int d = (int)(i % pad);
+  out[i] = d < sub ? h_rn((float)((double)cb[w * sub + d] * ldexp(1.0, scale_exp))) : (uint16_t)0;
 }
 
 // ---- candidates -----------------------------------------------------------------------------
@@ -586,14 +590,19 @@ __device__ __forceinline__ uint32_t words2(uint32_t w, uint32_t hsel, int b) {
   return __builtin_amdgcn_perm(hsel, w, sel);
 }
 
-// The B fragment of chunk c: dims 8c .. 8c + 7 of the lane half's decoded row.
+// B fragments of the lane half's decoded row: chunk c is its dims 8c .. 8c + 7.
+// Chunks are decoded kDecode<S> at a time, the fewest that hold whole codewords:
+// one for 2, 4 or 8 dims a code, three (24 dims) for 3 or 6.
+template <int S>
+constexpr int kDecode = S % 3 == 0 ? 3 : 1;
+__host__ __device__ constexpr int screen_pad(int sub) { return sub == 3 ? 4 : sub == 6 ? 8 : sub; }
 template <int D, int M>
-__device__ __forceinline__ f16x8 decode_chunk(const uint16_t* cbs, const uint32_t (&cw)[M / 8], uint32_t hsel,
-                                               int c) {
+__device__ __forceinline__ void decode_chunks(const uint16_t* cbs, const uint32_t (&cw)[M / 8], uint32_t hsel, int c,
+                                              f16x8 (&out)[kDecode<D / M>]) {
   constexpr int S = D / M;
-  constexpr int SUB = 512 * S;  // bytes per subspace of the fp16 codebook
+  constexpr int SUB = 512 * screen_pad(S);  // bytes per subspace of the fp16 codebook
   const char* base = reinterpret_cast<const char*>(cbs);
-  uint32_t f[4];
+  uint32_t f[4 * kDecode<S>];
   if constexpr (S == 4) {
     const uint32_t wd = words2(cw[c >> 1], hsel, 2 * (c & 1));
     const uint32_t a0 = (wd & 0xFFFFu) << 3, a1 = (wd >> 16) << 3;
@@ -605,15 +614,43 @@ __device__ __forceinline__ f16x8 decode_chunk(const uint16_t* cbs, const uint32_
     const uint32_t a0 = (wd & 0xFFFFu) << 4;
     const uint4 e = *reinterpret_cast<const uint4*>(base + a0 + c * SUB);
     f[0] = e.x; f[1] = e.y; f[2] = e.z; f[3] = e.w;
+  } else if constexpr (S == 6) {
+    // chunks c .. c + 2 are codes 4 c / 3 .. + 3, three dwords each
+    const int j = 4 * (c / 3);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t wd = words2(cw[j >> 2], hsel, 2 * i);
+      const uint4 e0 = *reinterpret_cast<const uint4*>(base + ((wd & 0xFFFFu) << 4) + (j + 2 * i) * SUB);
+      const uint4 e1 = *reinterpret_cast<const uint4*>(base + ((wd >> 16) << 4) + (j + 2 * i + 1) * SUB);
+      f[6 * i] = e0.x; f[6 * i + 1] = e0.y; f[6 * i + 2] = e0.z;
+      f[6 * i + 3] = e1.x; f[6 * i + 4] = e1.y; f[6 * i + 5] = e1.z;
+    }
+  } else if constexpr (S == 3) {
+    // chunks c .. c + 2 are codes 8 c / 3 .. + 7, two codes (x0 x1)(x2 0)(y0 y1)(y2 0)
+    // to three dwords (x0 x1)(x2 y0)(y1 y2)
+    const int j = 8 * (c / 3);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t wd = words2(cw[(j + 2 * i) >> 2], hsel, (2 * i) & 3);
+      const uint2 e0 = *reinterpret_cast<const uint2*>(base + ((wd & 0xFFFFu) << 3) + (j + 2 * i) * SUB);
+      const uint2 e1 = *reinterpret_cast<const uint2*>(base + ((wd >> 16) << 3) + (j + 2 * i + 1) * SUB);
+      f[3 * i] = e0.x;
+      f[3 * i + 1] = (e1.x << 16) | e0.y;
+      f[3 * i + 2] = __builtin_amdgcn_alignbit(e1.y, e1.x, 16);
+    }
   } else {
-    static_assert(S == 2, "screen: sub-dimension 2, 4 or 8");
+    static_assert(S == 2, "screen: sub-dimension 2, 3, 4, 6 or 8");
     const uint32_t w01 = words2(cw[c], hsel, 0), w23 = words2(cw[c], hsel, 2);
     f[0] = *reinterpret_cast<const uint32_t*>(base + ((w01 & 0xFFFFu) << 2) + (4 * c) * SUB);
     f[1] = *reinterpret_cast<const uint32_t*>(base + ((w01 >> 16) << 2) + (4 * c + 1) * SUB);
     f[2] = *reinterpret_cast<const uint32_t*>(base + ((w23 & 0xFFFFu) << 2) + (4 * c + 2) * SUB);
     f[3] = *reinterpret_cast<const uint32_t*>(base + ((w23 >> 16) << 2) + (4 * c + 3) * SUB);
   }
-  return __builtin_bit_cast(f16x8, f);
+#pragma unroll
+  for (int i = 0; i < kDecode<S>; ++i) {
+    const uint32_t g[4] = {f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]};
+    out[i] = __builtin_bit_cast(f16x8, g);
+  }
 }
 
 __device__ __forceinline__ f16x8 frag_of(uint32_t x, uint32_t y, uint32_t z, uint32_t w) {
@@ -659,7 +696,7 @@ __global__ __launch_bounds__(kSW * kWave) void screen_kernel(ScreenArgs a) {
   constexpr int NC = D / 16;  // main K chunks
   constexpr int HB = M / 2;   // code bytes per lane half
   static_assert(D % 32 == 0 && D <= 128, "screen: dim a multiple of 32, at most 128");
-  constexpr int kCbBytes = D * kPQK * 2;
+  constexpr int kCbBytes = M * screen_pad(D / M) * kPQK * 2;
   constexpr int kWaveWords = ROUND == 1 ? 0 : 2 * kCandBuf;  // staged (row, vector position) pairs
   constexpr int kRowWords = ROUND == 1 ? kQB : 3 * kQB;        // each row's query (+ round 2: count or first slot, t)
   constexpr int kPreOff = kCbBytes + kSW * (kWaveWords + kRowWords) * 4;
@@ -851,8 +888,13 @@ __global__ __launch_bounds__(kSW * kWave) void screen_kernel(ScreenArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[c], decode_chunk<D, M>(cbs, cw, hsel, c), acc, 0, 0, 0);
+      for (int c = 0; c < NC; c += kDecode<D / M>) {
+        f16x8 b[kDecode<D / M>];
+        decode_chunks<D, M>(cbs, cw, hsel, c, b);
+#pragma unroll
+        for (int i = 0; i < kDecode<D / M>; ++i)
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[c + i], b[i], acc, 0, 0, 0);
+      }
       const bool col = j0 + li < je;
       const uint4 bh = h == 0 ? (col ? bx : make_uint4(0u, 0u, 0u, 0u)) : (col ? h1_real : h1_pad);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(Aex, frag_of(bh.x, bh.y, bh.z, bh.w), acc, 0, 0, 0);
@@ -1136,15 +1178,17 @@ int64_t screen_gmin_words(int nq) {
 }
 
 bool screen_supported(int dim, int m) {
-  return (dim == 128 && (m == 16 || m == 32 || m == 64)) || (dim == 96 && m == 48);
+  return (dim == 128 && (m == 16 || m == 32 || m == 64)) || (dim == 96 && (m == 16 || m == 32 || m == 48));
 }
+
+size_t screen_codebook_words(int dim, int m) { return (size_t)m * kPQK * screen_pad(dim / m); }
 
 
 fgpu_status launch_screen_prep(const float* codebook, int m, int sub, int scale_exp, const uint8_t* codes,
                                int64_t total, uint16_t* cb16, uint4* vext, unsigned int* xmax_bits, hipStream_t s) {
-  const int64_t ncb = (int64_t)m * kPQK * sub;
-  hipLaunchKernelGGL(cb_f16_kernel, dim3((unsigned)((ncb + 255) / 256)), dim3(256), 0, s, codebook, ncb, scale_exp,
-                     cb16);
+  const int64_t ncb = (int64_t)screen_codebook_words(m * sub, m);
+  hipLaunchKernelGGL(cb_f16_kernel, dim3((unsigned)((ncb + 255) / 256)), dim3(256), 0, s, codebook, (int64_t)m * kPQK,
+                     sub, screen_pad(sub), scale_exp, cb16);
   FGPU_HIP(hipMemsetAsync(xmax_bits, 0, sizeof(unsigned int), s));
   if (total > 0)
     hipLaunchKernelGGL(screen_prep_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, codebook, m, sub,
@@ -1171,6 +1215,8 @@ fgpu_status launch_screen(int dim, int m, const ScreenArgs& a, hipStream_t s) {
   if (dim == 128 && m == 16) return launch_screen_dm<128, 16>(a, s);
   if (dim == 128 && m == 64) return launch_screen_dm<128, 64>(a, s);
   if (dim == 96 && m == 48) return launch_screen_dm<96, 48>(a, s);
+  if (dim == 96 && m == 32) return launch_screen_dm<96, 32>(a, s);
+  if (dim == 96 && m == 16) return launch_screen_dm<96, 16>(a, s);
   return set_error(FGPU_ERR_UNSUPPORTED, "screen: unsupported (dim, pq_m)");
 }
 

@@ -417,3 +417,31 @@ def test_small_batches_split_their_probes(dim, m, nq, nprobe, k):
         g.replay()
         assert np.array_equal(_host(out[0]), want[0]) and np.array_equal(_bits(_host(out[1])), _bits(want[1]))
     idx.close()
+
+
+@pytest.mark.parametrize("m,k,nq,nprobe", [(16, 10, 3072, 12), (32, 32, 3101, 12), (32, 5, 3072, 1), (16, 50, 800, 70),
+                                           (32, 64, 768, 66)])
+def test_screen_codes_of_3_and_6_dims(m, k, nq, nprobe):
+    """96 dims in 32 or 16 codes: codewords of 3 or 6 dims, padded in the screen's codebook and decoded three
+    fragments at a time (large batches, or more probes than the flow kernel takes)."""
+    _say(f"screen 96 dims m={m} k={k} nq={nq} nprobe={nprobe}")
+    offs, ids, codes, cent, cb = _gmm_index(96, m, 100, 24000, seed=m + k)
+    idx = fg.Index.from_arrays(96, m, offs, ids, codes, cent, cb)
+    assert idx.screen_ready
+    q = fg.gen_gmm(nq, 96, 32, seed=m + k, set=1, sig_lo=0.08)
+    st = _check(idx, q, cent, cb, offs, ids, codes, nprobe, k)
+    assert st["queries_with_threshold"] >= nq * 8 // 10 and st["queries_to_lut_kernel"] <= nq // 2
+    idx.close()
+
+
+@pytest.mark.parametrize("dim,m,nq,k", [(128, 32, 256, 10), (128, 32, 257, 10), (128, 16, 257, 33), (128, 16, 2049, 33),
+                                        (96, 16, 3071, 10), (96, 32, 3072, 33), (96, 16, 767, 10)])
+def test_search_route_edges(dim, m, nq, k):
+    """Batch sizes on both sides of the lines between the flow kernel and the screen (an index of 66,000 vectors):
+    the same results either way."""
+    _say(f"route edges dim={dim} m={m} nq={nq} k={k}")
+    offs, ids, codes, cent, cb = _gmm_index(dim, m, 128, 66000, seed=dim + m)
+    idx = fg.Index.from_arrays(dim, m, offs, ids, codes, cent, cb)
+    q = fg.gen_gmm(nq, dim, 32, seed=dim + m, set=1, sig_lo=0.08)
+    _check(idx, q, cent, cb, offs, ids, codes, 70 if nq == 767 else 10, k, screened=False)
+    idx.close()
