@@ -377,7 +377,9 @@ __global__ __launch_bounds__(kPPBlock) void pp_update_kernel(const float* __rest
                                                              float* __restrict__ d2, const int* __restrict__ shift,
                                                              uint64_t* __restrict__ w, uint64_t* __restrict__ part,
                                                              int32_t* __restrict__ asg, const float* __restrict__ cc,
-                                                             int j) {
+                                                             int j, const int32_t* __restrict__ picked,
+                                                             uint8_t* __restrict__ chosen) {
+  if (picked && blockIdx.x == 0 && threadIdx.x == 0) chosen[*picked] = 1;  // the pick itself must not see it
   const int64_t i = (int64_t)blockIdx.x * kPPBlock + threadIdx.x;
   uint64_t wi = 0;
   if (i < n) {
@@ -418,90 +420,104 @@ __global__ __launch_bounds__(kPPBlock) void pp_update_kernel(const float* __rest
   }
 }
 
-// The same update for a compile-time dim: each lane still owns one row and
-// keeps the sequential fused chain, but the row arrives as D/4 16-byte loads
-// that are all issued before the chain starts, instead of D dependent scalar
-// loads.
+// The same update for rows of whole 128-byte lines.  A workgroup takes the
+// kPPBlock rows of one part sum, four a thread; the rows that must compute are
+// packed per wave and read 64 at a time, eight lanes a row (wave_rows_l2: the
+// same chain, on c - x).  The rows read bound it: of 500k rows of 128 dims in
+// 1000 clusters a pass computes a third on average, 14.9 us, 10.4 us in the
+// median.  (One lane a row, 1024 threads and 128 registers of row: 15.0 us; 512
+// threads with half the hand-over buffer a wave: 15.6 us.)
+constexpr int kPPThreads = 256;
 template <int D>
-__global__ __launch_bounds__(kPPBlock) void pp_update_vec_kernel(const float* __restrict__ x, int64_t n,
-                                                                 const float* __restrict__ c, int init,
-                                                                 float* __restrict__ d2, const int* __restrict__ shift,
-                                                                 uint64_t* __restrict__ w, uint64_t* __restrict__ part,
-                                                                 int32_t* __restrict__ asg,
-                                                                 const float* __restrict__ cc, int jc) {
-  static_assert(D % 4 == 0, "16-byte row loads");
+__global__ __launch_bounds__(kPPThreads) void pp_update_rows_kernel(
+    const float* __restrict__ x, int64_t n, const float* __restrict__ c, int init, float* __restrict__ d2,
+    const int* __restrict__ shift, uint64_t* __restrict__ w, uint64_t* __restrict__ part, int32_t* __restrict__ asg,
+    const float* __restrict__ cc, int jc, const int32_t* __restrict__ picked, uint8_t* __restrict__ chosen) {
+  constexpr int kPer = kPPBlock / kPPThreads, kWaves = kPPThreads / kWave;
+  __shared__ __align__(16) float tr_s[kWaves][row_tr_floats()];
   __shared__ float cs[D];
-  for (int d = threadIdx.x; d < D; d += kPPBlock) cs[d] = c[d];
+  __shared__ int list_s[kWaves][kPer * kWave];
+  __shared__ float dist_s[kWaves][kPer * kWave];
+  __shared__ uint64_t s[kWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (picked && blockIdx.x == 0 && tid == 0) chosen[*picked] = 1;  // the pick itself must not see it
+  for (int d = tid; d < D; d += kPPThreads) cs[d] = c[d];
   __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * kPPBlock + threadIdx.x;
-  uint64_t wi = 0;
-  if (i < n) {
-    const float old = init ? 0.0f : d2[i];
-    float v2 = old;
-    bool moved = false;
-    if (init || pp_needs(init ? nullptr : asg, cc, i, old)) {
-      const float4* xi = reinterpret_cast<const float4*>(x + i * D);
-      float4 v[D / 4];
+  const int64_t b0 = (int64_t)blockIdx.x * kPPBlock;
+  int* list = list_s[wave];
+  float* dist = dist_s[wave];
+  float old[kPer];
+  int at[kPer];  // the row's place in the wave's list, -1: none
+  int m = 0;
 #pragma unroll
-      for (int j = 0; j < D / 4; ++j) v[j] = xi[j];
-      float acc = 0.0f;
+  for (int k = 0; k < kPer; ++k) {
+    const int64_t i = b0 + k * kPPThreads + tid;
+    old[k] = i < n && !init ? d2[i] : 0.0f;
+    const bool f = i < n && (init || pp_needs(asg, cc, i, old[k]));
+    const uint64_t bm = __ballot(f);
+    at[k] = f ? m + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u))
+              : -1;
+    if (f) list[at[k]] = (int)i;
+    m += __popcll(bm);
+  }
+  wave_lds_order();
+  for (int p = 0; p < m; p += kWave)
+    dist[p + lane] = wave_rows_l2<D, kWave, 1>(x, list[min(p + lane, m - 1)], cs, tr_s[wave]);
+  wave_lds_order();
+  uint64_t sum = 0;
 #pragma unroll
-      for (int j = 0; j < D / 4; ++j) {
-        float df = v[j].x - cs[4 * j];
-        acc = __builtin_fmaf(df, df, acc);
-        df = v[j].y - cs[4 * j + 1];
-        acc = __builtin_fmaf(df, df, acc);
-        df = v[j].z - cs[4 * j + 2];
-        acc = __builtin_fmaf(df, df, acc);
-        df = v[j].w - cs[4 * j + 3];
-        acc = __builtin_fmaf(df, df, acc);
-      }
-      moved = init || acc < old;
-      v2 = moved ? acc : old;
-    }
+  for (int k = 0; k < kPer; ++k) {
+    const int64_t i = b0 + k * kPPThreads + tid;
+    if (i >= n) continue;
+    const float acc = at[k] >= 0 ? dist[at[k]] : 0.0f;
+    const bool moved = at[k] >= 0 && (init || acc < old[k]);
+    const float v = moved ? acc : old[k];
     if (moved) {
-      d2[i] = v2;
+      d2[i] = v;
       if (asg) asg[i] = jc;
     }
     if (shift) {
-      wi = (uint64_t)__double2ll_rn(ldexp((double)v2, *shift));
+      const uint64_t wi = (uint64_t)__double2ll_rn(ldexp((double)v, *shift));
       if (moved || !asg) w[i] = wi;
+      sum += wi;
     }
   }
   if (shift) {
-    __shared__ uint64_t s[kPPBlock / kWave];
-    uint64_t t = wi;
 #pragma unroll
-    for (int m = 32; m > 0; m >>= 1) t += __shfl_xor(t, m, kWave);
-    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = t;
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+    if (lane == 0) s[wave] = sum;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
       uint64_t tot = 0;
-      for (int j = 0; j < kPPBlock / kWave; ++j) tot += s[j];
+      for (int k = 0; k < kWaves; ++k) tot += s[k];
       part[blockIdx.x] = tot;
     }
   }
 }
 
-// One pass of the d2 update: the vectorised kernel for the common dims (rows
-// 16-byte aligned), the generic one otherwise.
+// One pass of the d2 update: the row kernel for the common dims (rows 16-byte
+// aligned), the generic one otherwise.
 // asg == nullptr: every row computes (the first passes); otherwise the skip
-// above applies (cc filled for centre j).
+// above applies (cc filled for centre j).  picked: the row of centre j, which
+// the pass marks in chosen (nullptr: already marked).
 fgpu_status pp_update(const float* x, int64_t n, int dim, const float* c, int init, float* d2, const int* shift,
-                      uint64_t* w, uint64_t* part, int nb, int32_t* asg, const float* cc, int j, hipStream_t s) {
+                      uint64_t* w, uint64_t* part, int nb, int32_t* asg, const float* cc, int j,
+                      const int32_t* picked, uint8_t* chosen, hipStream_t s) {
   const bool vec = ((uintptr_t)x & 15) == 0;
-  if (vec && dim == 128)
-    hipLaunchKernelGGL(pp_update_vec_kernel<128>, dim3(nb), dim3(kPPBlock), 0, s, x, n, c, init, d2, shift, w, part,
-                       asg, cc, j);
-  else if (vec && dim == 96)
-    hipLaunchKernelGGL(pp_update_vec_kernel<96>, dim3(nb), dim3(kPPBlock), 0, s, x, n, c, init, d2, shift, w, part,
-                       asg, cc, j);
-  else if (vec && dim == 64)
-    hipLaunchKernelGGL(pp_update_vec_kernel<64>, dim3(nb), dim3(kPPBlock), 0, s, x, n, c, init, d2, shift, w, part,
-                       asg, cc, j);
-  else
-    hipLaunchKernelGGL(pp_update_kernel, dim3(nb), dim3(kPPBlock), 0, s, x, n, dim, c, init, d2, shift, w, part, asg,
-                       cc, j);
+#define FGPU_PP(D)                                                                                                   \
+  if (vec && dim == D) {                                                                                             \
+    hipLaunchKernelGGL(pp_update_rows_kernel<D>, dim3(nb), dim3(kPPThreads), 0, s, x, n, c, init, d2, shift, w, part, \
+                       asg, cc, j, picked, chosen);                                                                  \
+    FGPU_HIP(hipGetLastError());                                                                                     \
+    return FGPU_OK;                                                                                                  \
+  }
+  FGPU_PP(128)
+  FGPU_PP(96)
+  FGPU_PP(64)
+  FGPU_PP(32)
+#undef FGPU_PP
+  hipLaunchKernelGGL(pp_update_kernel, dim3(nb), dim3(kPPBlock), 0, s, x, n, dim, c, init, d2, shift, w, part, asg, cc, j,
+                     picked, chosen);
   FGPU_HIP(hipGetLastError());
   return FGPU_OK;
 }
@@ -526,111 +542,101 @@ __global__ __launch_bounds__(1024) void pp_shift_kernel(const float* __restrict_
   }
 }
 
-// Pick the next centre: smallest i with inclusive prefix(w) > u, u = r_j % total.
-// One workgroup; state[0] = chosen row.  chosen[] marks picked rows for the
-// all-zero fallback.
-// Then (cent != nullptr) take the picked row as centre j.
-__global__ __launch_bounds__(1024) void pp_pick_kernel(const uint64_t* __restrict__ w, const uint64_t* __restrict__ part,
-                                                       int nblocks, int64_t n, uint64_t seed, int j,
-                                                       uint8_t* __restrict__ chosen, int32_t* __restrict__ rows,
-                                                       const float* __restrict__ x, int dim, float* __restrict__ cent) {
-  __shared__ uint64_t s_tot;
-  __shared__ uint64_t s_u;
-  __shared__ int64_t s_pick;
-  __shared__ uint64_t s_before;
-  __shared__ int s_blk;
-  const int tid = threadIdx.x;
-  // Total and the block holding u: chunked parallel scan over the block sums.
-  __shared__ uint64_t sc[kPPBlock];
-  if (tid == 0) { s_tot = 0; s_blk = -1; s_pick = -1; s_before = 0; }
-  __syncthreads();
-  for (int base = 0; base < nblocks; base += kPPBlock) {
-    const uint64_t v = base + tid < nblocks ? part[base + tid] : 0;
-    sc[tid] = v;
-    __syncthreads();
-    for (int o = 1; o < kPPBlock; o <<= 1) {
-      const uint64_t t = tid >= o ? sc[tid - o] : 0;
-      __syncthreads();
-      sc[tid] += t;
-      __syncthreads();
-    }
-    if (tid == kPPBlock - 1) s_before = s_tot;  // running total before this chunk
-    __syncthreads();
-    const uint64_t chunk_before = s_before;
-    __syncthreads();
-    if (tid == kPPBlock - 1) s_tot = chunk_before + sc[tid];
-    __syncthreads();
+// Inclusive scan of one u64 a thread over a workgroup of kPPBlock threads.
+__device__ __forceinline__ uint64_t pp_scan(uint64_t v, uint64_t* wsum) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint64_t t = __shfl_up(v, o, kWave);
+    if (lane >= o) v += t;
   }
-  if (tid == 0 && s_tot != 0) s_u = mix64(seed ^ mix64(7) ^ mix64(0x100000000ull + (uint64_t)j)) % s_tot;
+  __syncthreads();  // wsum's last readers
+  if (lane == kWave - 1) wsum[wave] = v;
   __syncthreads();
-  if (s_tot != 0) {
-    uint64_t acc = 0;
-    for (int base = 0; base < nblocks; base += kPPBlock) {
-      const uint64_t v = base + tid < nblocks ? part[base + tid] : 0;
-      sc[tid] = v;
-      __syncthreads();
-      for (int o = 1; o < kPPBlock; o <<= 1) {
-        const uint64_t t = tid >= o ? sc[tid - o] : 0;
-        __syncthreads();
-        sc[tid] += t;
-        __syncthreads();
-      }
-      const uint64_t incl = acc + sc[tid], excl = incl - v;
-      if (base + tid < nblocks && excl <= s_u && s_u < incl) { s_blk = base + tid; s_before = excl; }
-      acc += sc[kPPBlock - 1];
-      __syncthreads();
-    }
-  }
-  __syncthreads();
-  if (tid == 0 && s_blk < 0) { s_blk = 0; s_before = 0; }  // unreachable when u < total; keeps indices in range
-  __syncthreads();
-  if (s_tot == 0) {
-    if (tid == 0) {
-      int64_t pick = 0;
-      for (int64_t i = 0; i < n; ++i)
-        if (!chosen[i]) { pick = i; break; }
-      s_pick = pick;
-    }
-  } else {
-    // Inside the block: inclusive scan of its 1024 weights.
-    const int64_t i = (int64_t)s_blk * kPPBlock + tid;
-    const uint64_t wi = i < n ? w[i] : 0;
-    sc[tid] = wi;
-    __syncthreads();
-    for (int o = 1; o < kPPBlock; o <<= 1) {
-      uint64_t t = tid >= o ? sc[tid - o] : 0;
-      __syncthreads();
-      sc[tid] += t;
-      __syncthreads();
-    }
-    const uint64_t incl = s_before + sc[tid];
-    const uint64_t excl = incl - wi;
-    if (i < n && excl <= s_u && s_u < incl) s_pick = i;
-    __syncthreads();
-    // s_u lies inside block s_blk by construction; the fallback only keeps the row in range.
-    if (tid == 0 && s_pick < 0) s_pick = (int64_t)s_blk * kPPBlock;
-  }
-  __syncthreads();
-  const int64_t r = s_pick;
-  if (tid == 0) rows[j] = (int32_t)r;
-  if (!cent) return;
-  for (int d = tid; d < dim; d += kPPBlock) cent[(int64_t)j * dim + d] = x[r * dim + d];
-  if (tid == 0) chosen[r] = 1;
+  uint64_t before = 0;
+#pragma unroll
+  for (int i = 0; i < kPPBlock / kWave; ++i) before += i < wave ? wsum[i] : 0;
+  return v + before;
 }
 
-// cc[a] = ||c_j - c_a||^2 for every earlier centre a < j: one wave per centre,
-// lanes over dimensions.  Only the skip bound reads cc, and that bound holds
-// for any summation order.
-__global__ __launch_bounds__(256) void pp_cc_kernel(const float* __restrict__ cent, int dim, int j,
-                                                    float* __restrict__ cc) {
-  const int a = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
+// Pick the next centre: smallest i with inclusive prefix(w) > u, u = r_j % total
+// (every weight zero: the lowest row not yet chosen), and its squared distance
+// to every earlier centre, cc[a] = ||c_j - c_a||^2, which only the update's skip
+// bound reads (any summation order).  Every workgroup finds the same pick and
+// takes 16 earlier centres, a wave each, lanes over dimensions; the first one
+// writes the row and the centre.  One launch: the pick (two scans by wave
+// shuffles) and the distances took 8.3 + 3.2 us as two kernels and a
+// launch more, 6.7 us now (500k rows, 1024 centres).
+__global__ __launch_bounds__(kPPBlock) void pp_pick_kernel(const uint64_t* __restrict__ w,
+                                                           const uint64_t* __restrict__ part, int nblocks, int64_t n,
+                                                           uint64_t seed, int j, const uint8_t* __restrict__ chosen,
+                                                           int32_t* __restrict__ rows, const float* __restrict__ x,
+                                                           int dim, float* __restrict__ cent, float* __restrict__ cc) {
+  __shared__ uint64_t wsum[kPPBlock / kWave];
+  __shared__ uint64_t s_before, s_tot;
+  __shared__ int s_blk;
+  __shared__ int64_t s_pick;
+  const int tid = threadIdx.x;
+  if (tid == 0) {
+    s_blk = -1;
+    s_pick = -1;
+    s_before = 0;
+  }
+  uint64_t tot = 0, first = 0;  // first: this thread's part sum of the first chunk, scanned
+  for (int base = 0; base < nblocks; base += kPPBlock) {
+    const uint64_t incl = pp_scan(base + tid < nblocks ? part[base + tid] : 0, wsum);
+    if (base == 0) first = incl;
+    if (tid == kPPBlock - 1) s_tot = incl;
+    __syncthreads();
+    tot += s_tot;
+    __syncthreads();
+  }
+  if (tot != 0) {
+    const uint64_t u = mix64(seed ^ mix64(7) ^ mix64(0x100000000ull + (uint64_t)j)) % tot;
+    uint64_t acc = 0;  // the chunks before this one
+    for (int base = 0; base < nblocks; base += kPPBlock) {
+      const uint64_t v = base + tid < nblocks ? part[base + tid] : 0;
+      const uint64_t in = base == 0 ? first : pp_scan(v, wsum);
+      const uint64_t incl = acc + in, excl = incl - v;
+      if (base + tid < nblocks && excl <= u && u < incl) {
+        s_blk = base + tid;
+        s_before = excl;
+      }
+      if (base + kPPBlock < nblocks) {
+        if (tid == kPPBlock - 1) s_tot = in;
+        __syncthreads();
+        acc += s_tot;
+        __syncthreads();
+      }
+    }
+    __syncthreads();
+    const int64_t i = (int64_t)max(s_blk, 0) * kPPBlock + tid;  // (a block holds u by construction)
+    const uint64_t wi = i < n ? w[i] : 0;
+    const uint64_t incl = s_before + pp_scan(wi, wsum), excl = incl - wi;
+    if (i < n && excl <= u && u < incl) s_pick = i;
+    __syncthreads();
+    if (tid == 0 && s_pick < 0) s_pick = (int64_t)max(s_blk, 0) * kPPBlock;
+  } else if (tid == 0) {
+    int64_t pick = 0;
+    for (int64_t i = 0; i < n; ++i)
+      if (!chosen[i]) {
+        pick = i;
+        break;
+      }
+    s_pick = pick;
+  }
+  __syncthreads();
+  const float* xr = x + s_pick * dim;
+  if (blockIdx.x == 0) {
+    if (tid == 0) rows[j] = (int32_t)s_pick;
+    for (int d = tid; d < dim; d += kPPBlock) cent[(int64_t)j * dim + d] = xr[d];
+  }
+  const int a = blockIdx.x * (kPPBlock / kWave) + (tid >> 6), lane = tid & 63;
   if (a >= j) return;
-  const float* cj = cent + (size_t)j * dim;
   const float* ca = cent + (size_t)a * dim;
   float acc = 0.0f;
-  for (int d = lane; d < dim; d += 64) {
-    const float df = cj[d] - ca[d];
+  for (int d = lane; d < dim; d += kWave) {
+    const float df = xr[d] - ca[d];
     acc = __builtin_fmaf(df, df, acc);
   }
 #pragma unroll
@@ -854,19 +860,19 @@ fgpu_status launch_kmeans_pp(const float* x, int64_t n, int dim, int k, uint64_t
   FGPU_HIP(hipMemsetAsync(chosen, 0, n, s));
   hipLaunchKernelGGL(pp_first_kernel, dim3(1), dim3(1), 0, s, n, seed, rows, chosen);
   hipLaunchKernelGGL(pp_take_kernel, dim3(1), dim3(256), 0, s, x, dim, rows, 0, cent, chosen);
-  FGPU_TRY(pp_update(x, n, dim, cent, 1, d2, nullptr, w, part, nb, asg, cc, 0, s));  // asg := 0
+  FGPU_TRY(pp_update(x, n, dim, cent, 1, d2, nullptr, w, part, nb, asg, cc, 0, nullptr, chosen, s));  // asg := 0
   hipLaunchKernelGGL(pp_shift_kernel, dim3(1), dim3(1024), 0, s, d2, n, shift);
   FGPU_HIP(hipGetLastError());
   // weights for round 1 from the initial d2 (every row: no skip yet)
-  FGPU_TRY(pp_update(x, n, dim, cent, 0, d2, shift, w, part, nb, nullptr, cc, 0, s));
+  FGPU_TRY(pp_update(x, n, dim, cent, 0, d2, shift, w, part, nb, nullptr, cc, 0, nullptr, chosen, s));
   for (int j = 1; j < k; ++j) {
-    // pick and take the row as centre j in one workgroup
-    hipLaunchKernelGGL(pp_pick_kernel, dim3(1), dim3(kPPBlock), 0, s, w, part, nb, n, seed, j, chosen, rows, x, dim,
-                       cent);
-    if (j + 1 < k) {
-      hipLaunchKernelGGL(pp_cc_kernel, dim3((unsigned)((j + 3) / 4)), dim3(256), 0, s, cent, dim, j, cc);
-      FGPU_TRY(pp_update(x, n, dim, cent + (size_t)j * dim, 0, d2, shift, w, part, nb, asg, cc, j, s));
-    }
+    // the pick, the row as centre j and its distances to the earlier centres
+    // (those only if a pass follows)
+    const unsigned g = j + 1 < k ? (unsigned)((j + kPPBlock / kWave - 1) / (kPPBlock / kWave)) : 1u;
+    hipLaunchKernelGGL(pp_pick_kernel, dim3(g), dim3(kPPBlock), 0, s, w, part, nb, n, seed, j, chosen, rows, x, dim, cent,
+                       cc);
+    if (j + 1 < k)
+      FGPU_TRY(pp_update(x, n, dim, cent + (size_t)j * dim, 0, d2, shift, w, part, nb, asg, cc, j, rows + j, chosen, s));
   }
   FGPU_HIP(hipGetLastError());
   return FGPU_OK;

@@ -414,6 +414,25 @@ def test_kmeans_pp_seeding_bit_exact(n, dim, comp, k):
     assert np.array_equal(_bits(_host(cent)), _bits(want))
 
 
+@pytest.mark.parametrize("n,dim,k", [(1023, 32, 40), (1025, 64, 18), (1024, 96, 17), (70, 128, 70),
+                                     ((1 << 20) + 700, 32, 3)])
+def test_kmeans_pp_pick_and_update_edges(n, dim, k):
+    """Seeding at the edges of its kernels: part sums of 1024 rows, one row less
+    and one more, dims of one to four lines, more than 1024 part sums, centre
+    counts around a workgroup's 16, and (with 50 distinct rows) picks left when
+    every weight is zero, which take the lowest row not yet chosen.  The centres
+    are the oracle's bit for bit."""
+    _say(f"kmeans++ edges n={n} dim={dim} k={k}")
+    rng = np.random.default_rng(n + dim)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    if n == k:
+        x[50:] = x[: n - 50]
+    cent, _ = fg.kmeans_fit(torch.from_numpy(x).cuda(), k, 0, init_mode=1, seed=3, want_assign=False)
+    want, rows = oracle.kmeans_init_pp(x, k, 3)
+    assert len(set(rows.tolist())) == k
+    assert np.array_equal(_bits(_host(cent)), _bits(want))
+
+
 # --------------------------------------------------------------------------- PQ (A15, A16)
 def test_pq_train_matches_reference_fixture():
     _say("pq_train golden")
