@@ -1500,25 +1500,23 @@ fgpu_status fgpu_build_ivfpq_sampled(const float* dx, int64_t n, int dim, int nl
     FGPU_HIP(hipStreamSynchronize(s));
   }
   FGPU_TRY(fgpu_pq_train(dx, n, dim, pq_m, assign.p, cent.p, sample_size, pq_iters, cb.p, stream));
-  FGPU_TRY(fgpu_pq_encode(dx, n, dim, pq_m, assign.p, cent.p, cb.p, codes.p, stream));
-  std::vector<int32_t> ha(n);
-  std::vector<uint8_t> hc((size_t)n * pq_m);
-  FGPU_HIP(hipMemcpyAsync(ha.data(), assign.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost, s));
-  FGPU_HIP(hipMemcpyAsync(hc.data(), codes.p, hc.size(), hipMemcpyDeviceToHost, s));
+  // inverted lists in cluster order, ids ascending inside a list
+  // (build_global.cu:225-240); the codes are written in that order
+  DevBuf<int32_t> offs, ids, pos;
+  DevBuf<char> lws;
+  const size_t lb = list_order_ws_bytes(n, nlist);
+  FGPU_TRY(offs.alloc((size_t)nlist + 1));
+  FGPU_TRY(ids.alloc(n));
+  FGPU_TRY(pos.alloc(n));
+  FGPU_TRY(lws.alloc(lb));
+  FGPU_TRY(launch_list_order(assign.p, n, nlist, offs.p, ids.p, pos.p, lws.p, lb, s));
+  FGPU_TRY(launch_pq_encode(dx, n, dim, pq_m, assign.p, cent.p, cb.p, codes.p, s, 1, pos.p));
+  FGPU_HIP(hipMemcpyAsync(h_offsets, offs.p, sizeof(int32_t) * ((size_t)nlist + 1), hipMemcpyDeviceToHost, s));
+  FGPU_HIP(hipMemcpyAsync(h_ids, ids.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost, s));
+  FGPU_HIP(hipMemcpyAsync(h_codes, codes.p, (size_t)n * pq_m, hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipMemcpyAsync(h_centroids, cent.p, sizeof(float) * (size_t)nlist * dim, hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipMemcpyAsync(h_codebook, cb.p, sizeof(float) * (size_t)pq_m * kPQK * (dim / pq_m), hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipStreamSynchronize(s));
-  // inverted lists in cluster order, ids ascending inside a list (build_global.cu:225-240)
-  std::vector<int64_t> cnt(nlist + 1, 0);
-  for (int64_t i = 0; i < n; ++i) cnt[ha[i] + 1]++;
-  for (int l = 0; l < nlist; ++l) cnt[l + 1] += cnt[l];
-  for (int l = 0; l <= nlist; ++l) h_offsets[l] = (int32_t)cnt[l];
-  std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
-  for (int64_t i = 0; i < n; ++i) {
-    const int64_t pp = pos[ha[i]]++;
-    h_ids[pp] = (int32_t)i;
-    std::memcpy(h_codes + pp * pq_m, hc.data() + i * pq_m, pq_m);
-  }
   return FGPU_OK;
 }
 

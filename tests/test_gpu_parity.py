@@ -470,6 +470,20 @@ def test_build_ivfpq_bit_exact():
         assert np.array_equal(np.asarray(g).view(np.uint8), np.asarray(w).view(np.uint8)), name
 
 
+@pytest.mark.parametrize("n,nlist,distinct", [(256, 1, 256), (2048, 7, 2048), (2049, 300, 40), (6145, 33, 6145)])
+def test_build_lists_at_chunk_edges(n, nlist, distinct):
+    """The inverted lists at the edges of the 2048-row chunks they are sorted in: one list, a chunk of one row,
+    lists left empty by repeated rows."""
+    _say(f"build lists n={n} nlist={nlist}")
+    x = oracle.gen_gmm(n, 96, 8, seed=n, sig_lo=0.1)
+    x = np.ascontiguousarray(x[np.random.default_rng(n).integers(0, distinct, n)]) if distinct < n else x
+    kw = dict(kmeans_iters=2, init_mode=0, seed=3, pq_iters=1, sample_size=256)
+    got = fg.build_ivfpq(torch.from_numpy(x).cuda(), nlist, 16, **kw)
+    want = oracle.build_ivfpq(x, nlist, 16, **kw)
+    for g, w, name in zip(got, want, ["offsets", "ids", "codes", "centroids", "codebook"]):
+        assert np.array_equal(np.asarray(g).view(np.uint8), np.asarray(w).view(np.uint8)), name
+
+
 def test_config1_end_to_end_bit_exact():
     """BASELINE config 1 at full size: 100k x 128 (64-component mixture, sigma 0.1), 256 lists, PQ M=16,
     1000 queries, nprobe 16, k 10 -- index build and search, GPU against the oracle."""
