@@ -7,9 +7,11 @@
 #include <cstdio>
 #include <cstring>
 #include <fstream>
+#include <future>
 #include <numeric>
 #include <random>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -343,6 +345,55 @@ std::vector<int32_t> shuffled_prefix(int64_t n, int64_t k, std::mt19937& rng) {
   }
   return a;
 }
+
+// The rows PQ training draws, which depend on the sizes alone.
+struct PqSample {
+  int actual;                      // sample rows
+  std::vector<int32_t> rows, init; // the rows; each subspace's 256 initial ones, as places in rows
+  PqSample(int64_t n, int pq_m, int sample_size) : actual((int)std::min<int64_t>(sample_size, n)) {
+    // sample rows (pq_utils.h:91-97)
+    std::mt19937 rng(12345);
+    rows = shuffled_prefix(n, actual, rng);
+    // per-subspace initial rows (pq_utils.h:20-31, seed 1234+m)
+    // Each subspace's shuffle has its own generator: a few host threads.
+    init.resize((size_t)pq_m * kPQK);
+    const int nt = std::max(1, std::min(pq_m, 8));
+    std::vector<std::thread> th;
+    for (int t0 = 0; t0 < nt; ++t0)
+      th.emplace_back([&, t0] {
+        std::vector<int> ind(actual);
+        for (int sub = t0; sub < pq_m; sub += nt) {
+          std::iota(ind.begin(), ind.end(), 0);
+          std::mt19937 rng(1234 + sub);
+          std::shuffle(ind.begin(), ind.end(), rng);
+          std::copy(ind.begin(), ind.begin() + kPQK, init.begin() + (size_t)sub * kPQK);
+        }
+      });
+    for (auto& t : th) t.join();
+  }
+};
+
+fgpu_status pq_train_sampled(const float* dx, int dim, int pq_m, const int32_t* d_assign, const float* d_cent,
+                             const PqSample& sm, int iters, float* d_codebook, hipStream_t s) {
+  const int actual = sm.actual;
+  DevBuf<int32_t> drows, dinit, dassign;
+  DevBuf<float> res;
+  FGPU_TRY(drows.alloc(actual));
+  FGPU_TRY(dinit.alloc(sm.init.size()));
+  FGPU_TRY(dassign.alloc((size_t)actual * pq_m));
+  FGPU_TRY(res.alloc((size_t)actual * dim));
+  FGPU_HIP(hipMemcpyAsync(drows.p, sm.rows.data(), sizeof(int32_t) * actual, hipMemcpyHostToDevice, s));
+  FGPU_HIP(hipMemcpyAsync(dinit.p, sm.init.data(), sizeof(int32_t) * sm.init.size(), hipMemcpyHostToDevice, s));
+  FGPU_TRY(launch_pq_residuals(dx, dim, drows.p, actual, d_assign, d_cent, res.p, s));
+  FGPU_TRY(launch_pq_init(res.p, actual, dim, pq_m, dinit.p, d_codebook, s));
+  for (int it = 0; it < iters; ++it) {
+    FGPU_TRY(launch_pq_estep(res.p, actual, dim, pq_m, d_codebook, dassign.p, s));
+    FGPU_TRY(launch_pq_mstep(res.p, actual, dim, pq_m, dassign.p, d_codebook, s));
+  }
+  FGPU_HIP(hipStreamSynchronize(s));
+  return FGPU_OK;
+}
+
 
 int64_t topk_batch_rows(int64_t n, int nc) {
   const size_t budget = 256ull << 20;  // estimate tile budget per batch
@@ -1400,49 +1451,9 @@ fgpu_status fgpu_pq_train(const float* dx, int64_t n, int dim, int pq_m, const i
                           int sample_size, int iters, float* d_codebook, void* stream) {
   FGPU_CHECK(dx && d_assign && d_cent && d_codebook && n >= 1 && pq_m >= 1 && dim % pq_m == 0 && iters >= 0,
              FGPU_ERR_ARG, "pq_train: bad argument");
-  hipStream_t s = as_stream(stream);
-  // sample rows (pq_utils.h:91-97)
-  const int actual = (int)std::min<int64_t>(sample_size, n);
-  FGPU_CHECK(actual >= kPQK, FGPU_ERR_ARG, "pq_train: need at least 256 sample rows");
-  std::vector<int32_t> idx;
-  {
-    std::mt19937 rng(12345);
-    idx = shuffled_prefix(n, actual, rng);
-  }
-  // per-subspace initial rows (pq_utils.h:20-31, seed 1234+m)
-  // Each subspace's shuffle has its own generator: a few host threads.
-  std::vector<int32_t> init((size_t)pq_m * kPQK);
-  {
-    const int nt = std::max(1, std::min(pq_m, 8));
-    std::vector<std::thread> th;
-    for (int t0 = 0; t0 < nt; ++t0)
-      th.emplace_back([&, t0] {
-        std::vector<int> ind(actual);
-        for (int sub = t0; sub < pq_m; sub += nt) {
-          std::iota(ind.begin(), ind.end(), 0);
-          std::mt19937 rng(1234 + sub);
-          std::shuffle(ind.begin(), ind.end(), rng);
-          std::copy(ind.begin(), ind.begin() + kPQK, init.begin() + (size_t)sub * kPQK);
-        }
-      });
-    for (auto& t : th) t.join();
-  }
-  DevBuf<int32_t> drows, dinit, dassign;
-  DevBuf<float> res;
-  FGPU_TRY(drows.alloc(actual));
-  FGPU_TRY(dinit.alloc(init.size()));
-  FGPU_TRY(dassign.alloc((size_t)actual * pq_m));
-  FGPU_TRY(res.alloc((size_t)actual * dim));
-  FGPU_HIP(hipMemcpyAsync(drows.p, idx.data(), sizeof(int32_t) * actual, hipMemcpyHostToDevice, s));
-  FGPU_HIP(hipMemcpyAsync(dinit.p, init.data(), sizeof(int32_t) * init.size(), hipMemcpyHostToDevice, s));
-  FGPU_TRY(launch_pq_residuals(dx, dim, drows.p, actual, d_assign, d_cent, res.p, s));
-  FGPU_TRY(launch_pq_init(res.p, actual, dim, pq_m, dinit.p, d_codebook, s));
-  for (int it = 0; it < iters; ++it) {
-    FGPU_TRY(launch_pq_estep(res.p, actual, dim, pq_m, d_codebook, dassign.p, s));
-    FGPU_TRY(launch_pq_mstep(res.p, actual, dim, pq_m, dassign.p, d_codebook, s));
-  }
-  FGPU_HIP(hipStreamSynchronize(s));
-  return FGPU_OK;
+  FGPU_CHECK(std::min<int64_t>(sample_size, n) >= kPQK, FGPU_ERR_ARG, "pq_train: need at least 256 sample rows");
+  return pq_train_sampled(dx, dim, pq_m, d_assign, d_cent, PqSample(n, pq_m, sample_size), iters, d_codebook,
+                          as_stream(stream));
 }
 
 fgpu_status fgpu_pq_encode(const float* dx, int64_t n, int dim, int pq_m, const int32_t* d_assign,
@@ -1479,6 +1490,16 @@ fgpu_status fgpu_build_ivfpq_sampled(const float* dx, int64_t n, int dim, int nl
   FGPU_TRY(cb.alloc((size_t)pq_m * kPQK * (dim / pq_m)));
   FGPU_TRY(assign.alloc(n));
   FGPU_TRY(codes.alloc((size_t)n * pq_m));
+  // PQ training's sample is drawn on a host thread while the k-means runs (its
+  // arguments are checked here, the others where they are used)
+  const bool pq_ok = n >= 1 && pq_m >= 1 && dim % pq_m == 0 && std::min<int64_t>(sample_size, n) >= kPQK;
+  std::future<PqSample> sample;
+  if (pq_ok) {
+    try {
+      sample = std::async(std::launch::async, [=] { return PqSample(n, pq_m, sample_size); });
+    } catch (const std::system_error&) {  // no thread to be had: drawn below
+    }
+  }
   if (train_rows <= 0 || train_rows >= n) {
     FGPU_TRY(fgpu_kmeans_fit(dx, n, dim, nlist, kmeans_iters, init_mode, seed, cent.p, assign.p, stream));
   } else {
@@ -1499,7 +1520,9 @@ fgpu_status fgpu_build_ivfpq_sampled(const float* dx, int64_t n, int dim, int nl
     FGPU_TRY(fgpu_l2_topk(dx, n, cent.p, nlist, dim, 1, assign.p, dist.p, tws.p, tb, stream));
     FGPU_HIP(hipStreamSynchronize(s));
   }
-  FGPU_TRY(fgpu_pq_train(dx, n, dim, pq_m, assign.p, cent.p, sample_size, pq_iters, cb.p, stream));
+  FGPU_CHECK(pq_ok && pq_iters >= 0, FGPU_ERR_ARG, "build: pq_m must divide dim, pq_iters >= 0 and 256 sample rows or more");
+  FGPU_TRY(pq_train_sampled(dx, dim, pq_m, assign.p, cent.p, sample.valid() ? sample.get() : PqSample(n, pq_m, sample_size),
+                            pq_iters, cb.p, s));
   // inverted lists in cluster order, ids ascending inside a list
   // (build_global.cu:225-240); the codes are written in that order
   DevBuf<int32_t> offs, ids, pos;
