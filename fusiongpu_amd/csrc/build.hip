@@ -361,7 +361,7 @@ __global__ void pq_init_kernel(const float* __restrict__ res, int dim, int m, in
 template <int S>
 __global__ __launch_bounds__(256) void pq_estep_kernel(const float* __restrict__ res, int ns, int dim, int m,
                                                        const float* __restrict__ codebook,
-                                                       int32_t* __restrict__ assign_pq) {
+                                                       uint8_t* __restrict__ assign_pq, int stride) {
   __shared__ float cbs[kPQK * S];
   const int sub = blockIdx.y;
   for (int t = threadIdx.x; t < kPQK * S; t += blockDim.x) cbs[t] = codebook[(size_t)sub * kPQK * S + t];
@@ -382,30 +382,91 @@ __global__ __launch_bounds__(256) void pq_estep_kernel(const float* __restrict__
     }
     if (d < best) { best = d; bc = c; }
   }
-  assign_pq[(int64_t)sub * ns + i] = bc;
+  assign_pq[(size_t)sub * stride + i] = (uint8_t)bc;
 }
 
 // M-step (pq_utils.h:54-71): members of cluster c summed in double in
 // ascending row order, (float)(sum / count); an empty cluster keeps its
-// centre.  One wave per (cluster, subspace); lanes j < S own dimension j.
-__global__ __launch_bounds__(64) void pq_mstep_kernel(const float* __restrict__ res, int ns, int dim, int m, int S,
-                                                      const int32_t* __restrict__ assign_pq,
+// centre.  One wave per (cluster, subspace): it reads the subspace's
+// assignments a byte each, 1024 a step, lists the members in LDS in order, and
+// once 64 or more are
+// listed reads their values 64 rows at a time, all loads in flight together, before lane j < S adds dimension j's in order.  Scanning the
+// assignments bounds it (every cluster's wave reads them all, from L2).
+constexpr int kMStep = 1024, kMList = kMStep + 64;
+template <int S>
+__global__ __launch_bounds__(64) void pq_mstep_kernel(const float* __restrict__ res, int ns, int dim,
+                                                      const uint8_t* __restrict__ assign_pq, int stride,
                                                       float* __restrict__ codebook) {
+  __shared__ int list[kMList];
+  __shared__ float val[kWave * S];
   const int c = blockIdx.x, sub = blockIdx.y, lane = threadIdx.x;
-  const int32_t* as = assign_pq + (int64_t)sub * ns;
+  const uint4* as = reinterpret_cast<const uint4*>(assign_pq + (size_t)sub * stride);
+  const uint32_t c4 = (uint32_t)c * 0x01010101u;
+  const float* rs = res + sub * S;
   double acc = 0.0;
-  int cnt = 0;
-  for (int base = 0; base < ns; base += kWave) {
-    const int i = base + lane;
-    const bool hit = i < ns && as[i] == c;
-    uint64_t bm = __ballot(hit);
-    while (bm) {
-      const int b = __ffsll((unsigned long long)bm) - 1;
-      bm &= bm - 1;
-      if (lane < S) acc += (double)res[(int64_t)(base + b) * dim + sub * S + lane];
-      ++cnt;
+  int cnt = 0, m = 0;  // members so far, and of them those listed but not yet added
+  // adds the first r <= 64 listed rows from `at` on
+  auto add = [&](int at, int r) {
+    float v[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      const int e = min(lane + k * kWave, r * S - 1);
+      v[k] = rs[(int64_t)list[at + e / S] * dim + e % S];
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k) val[lane + k * kWave] = v[k];
+    wave_lds_order();
+    if (lane < S)
+#pragma unroll 8
+      for (int i = 0; i < r; ++i) acc += (double)val[i * S + lane];
+    wave_lds_order();
+  };
+  // the lane's 16 rows of a step: bit i set where row i is a member
+  auto members = [&](int base, uint4 w) {
+    const uint32_t v[4] = {w.x, w.y, w.z, w.w};
+    uint32_t hit = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t x = v[k] ^ c4;  // a zero byte: a member
+      const uint32_t z = ~(((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) & 0x80808080u;
+      hit |= (((z >> 7) * 0x01020408u) >> 24) << (4 * k);
+    }
+    const int left = ns - (base + 16 * lane);
+    return left >= 16 ? hit : left > 0 ? hit & ((1u << left) - 1u) : 0u;
+  };
+  const int last = stride / 16 - 1;
+  uint4 next = as[min(lane, last)];
+  for (int base = 0; base < ns; base += kMStep) {
+    uint32_t hit = members(base, next);
+    next = as[min((base + kMStep) / 16 + lane, last)];  // past the end: the last 16, unused
+    const int h = __popc(hit);
+    int incl = h;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int u = __shfl_up(incl, o, kWave);
+      if (lane >= o) incl += u;
+    }
+    const int all = __builtin_amdgcn_readlane(incl, kWave - 1);
+    int at = m + incl - h;
+    while (hit) {
+      list[at++] = base + 16 * lane + __ffs((int)hit) - 1;
+      hit &= hit - 1;
+    }
+    wave_lds_order();
+    m += all;
+    cnt += all;
+    if (m >= kWave) {  // at least 1024 free places after it
+      int i = 0;
+      for (; i + kWave <= m; i += kWave) add(i, kWave);
+      const int rest = m - i;
+      const int keep = lane < rest ? list[i + lane] : 0;
+      wave_lds_order();
+      if (lane < rest) list[lane] = keep;
+      wave_lds_order();
+      m = rest;
     }
   }
+  if (m > 0) add(0, m);
   if (lane < S && cnt > 0) codebook[((size_t)sub * kPQK + c) * S + lane] = (float)(acc / (double)cnt);
 }
 
@@ -919,28 +980,39 @@ fgpu_status launch_pq_init(const float* res, int nsample, int dim, int m, const 
   return launch1d(pq_init_kernel, (int64_t)m * kPQK * S, 256, s, res, dim, m, S, init_rows, codebook);
 }
 
-fgpu_status launch_pq_estep(const float* res, int ns, int dim, int m, const float* codebook, int32_t* assign_pq,
+// A subspace's assignments: ns bytes, rounded up to whole 16-byte loads.
+static int pq_stride(int ns) { return (ns + 15) / 16 * 16; }
+size_t pq_assign_bytes(int ns, int m) { return (size_t)pq_stride(ns) * m; }
+
+fgpu_status launch_pq_estep(const float* res, int ns, int dim, int m, const float* codebook, uint8_t* assign_pq,
                             hipStream_t s) {
   const int S = dim / m;
   dim3 grid((unsigned)((ns + 255) / 256), (unsigned)m);
-#define FGPU_EST(SS)                                                                                   \
-  if (S == SS) {                                                                                       \
-    hipLaunchKernelGGL(pq_estep_kernel<SS>, grid, dim3(256), 0, s, res, ns, dim, m, codebook, assign_pq); \
-    FGPU_HIP(hipGetLastError());                                                                       \
-    return FGPU_OK;                                                                                    \
+#define FGPU_EST(SS)                                                                                     \
+  if (S == SS) {                                                                                         \
+    hipLaunchKernelGGL(pq_estep_kernel<SS>, grid, dim3(256), 0, s, res, ns, dim, m, codebook, assign_pq, \
+                       pq_stride(ns));                                                                   \
+    FGPU_HIP(hipGetLastError());                                                                         \
+    return FGPU_OK;                                                                                      \
   }
   FGPU_EST(1) FGPU_EST(2) FGPU_EST(3) FGPU_EST(4) FGPU_EST(6) FGPU_EST(8) FGPU_EST(16)
 #undef FGPU_EST
   return set_error(FGPU_ERR_UNSUPPORTED, "pq_estep: unsupported sub-dimension");
 }
 
-fgpu_status launch_pq_mstep(const float* res, int ns, int dim, int m, const int32_t* assign_pq, float* codebook,
+fgpu_status launch_pq_mstep(const float* res, int ns, int dim, int m, const uint8_t* assign_pq, float* codebook,
                             hipStream_t s) {
   const int S = dim / m;
-  FGPU_CHECK(S <= kWave, FGPU_ERR_UNSUPPORTED, "pq_mstep: sub-dimension above 64");
-  hipLaunchKernelGGL(pq_mstep_kernel, dim3(kPQK, (unsigned)m), dim3(64), 0, s, res, ns, dim, m, S, assign_pq, codebook);
-  FGPU_HIP(hipGetLastError());
-  return FGPU_OK;
+#define FGPU_MST(SS)                                                                                                  \
+  if (S == SS) {                                                                                                      \
+    hipLaunchKernelGGL(pq_mstep_kernel<SS>, dim3(kPQK, (unsigned)m), dim3(kWave), 0, s, res, ns, dim, assign_pq,      \
+                       pq_stride(ns), codebook);                                                                      \
+    FGPU_HIP(hipGetLastError());                                                                                      \
+    return FGPU_OK;                                                                                                   \
+  }
+  FGPU_MST(1) FGPU_MST(2) FGPU_MST(3) FGPU_MST(4) FGPU_MST(6) FGPU_MST(8) FGPU_MST(16)
+#undef FGPU_MST
+  return set_error(FGPU_ERR_UNSUPPORTED, "pq_mstep: unsupported sub-dimension");
 }
 
 size_t kmeans_pp_ws_bytes(int64_t n, int k) {

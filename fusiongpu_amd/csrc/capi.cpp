@@ -376,11 +376,12 @@ struct PqSample {
 fgpu_status pq_train_sampled(const float* dx, int dim, int pq_m, const int32_t* d_assign, const float* d_cent,
                              const PqSample& sm, int iters, float* d_codebook, hipStream_t s) {
   const int actual = sm.actual;
-  DevBuf<int32_t> drows, dinit, dassign;
+  DevBuf<int32_t> drows, dinit;
+  DevBuf<uint8_t> dassign;
   DevBuf<float> res;
   FGPU_TRY(drows.alloc(actual));
   FGPU_TRY(dinit.alloc(sm.init.size()));
-  FGPU_TRY(dassign.alloc((size_t)actual * pq_m));
+  FGPU_TRY(dassign.alloc(pq_assign_bytes(actual, pq_m)));
   FGPU_TRY(res.alloc((size_t)actual * dim));
   FGPU_HIP(hipMemcpyAsync(drows.p, sm.rows.data(), sizeof(int32_t) * actual, hipMemcpyHostToDevice, s));
   FGPU_HIP(hipMemcpyAsync(dinit.p, sm.init.data(), sizeof(int32_t) * sm.init.size(), hipMemcpyHostToDevice, s));

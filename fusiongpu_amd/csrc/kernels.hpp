@@ -446,9 +446,11 @@ fgpu_status launch_pq_residuals(const float* x, int dim, const int32_t* rows, in
                                 const int32_t* assign, const float* cent, float* res, hipStream_t s);
 fgpu_status launch_pq_init(const float* res, int nsample, int dim, int m, const int32_t* init_rows,
                            float* codebook, hipStream_t s);
+// assign_pq: pq_assign_bytes(nsample, m) bytes, 16-byte aligned.
+size_t pq_assign_bytes(int nsample, int m);
 fgpu_status launch_pq_estep(const float* res, int nsample, int dim, int m, const float* codebook,
-                            int32_t* assign_pq, hipStream_t s);
-fgpu_status launch_pq_mstep(const float* res, int nsample, int dim, int m, const int32_t* assign_pq,
+                            uint8_t* assign_pq, hipStream_t s);
+fgpu_status launch_pq_mstep(const float* res, int nsample, int dim, int m, const uint8_t* assign_pq,
                             float* codebook, hipStream_t s);
 // k-means++ seeding on the device (definition in oracle.cpp orc_kmeans_init_pp).
 fgpu_status launch_kmeans_pp(const float* x, int64_t n, int dim, int k, uint64_t seed, float* cent,

@@ -470,6 +470,21 @@ def test_build_ivfpq_bit_exact():
         assert np.array_equal(np.asarray(g).view(np.uint8), np.asarray(w).view(np.uint8)), name
 
 
+@pytest.mark.parametrize("ns,dim,m,distinct", [(256, 128, 128, 256), (1023, 96, 48, 3), (1025, 96, 32, 1025),
+                                               (2063, 128, 16, 2), (5000, 96, 16, 40), (3000, 128, 8, 700)])
+def test_pq_train_at_step_edges(ns, dim, m, distinct):
+    """Codebook training at the edges of the M step's 1024-row steps and 64-member rounds: every sub-dimension,
+    clusters of most rows (few distinct rows) and empty ones."""
+    _say(f"pq_train ns={ns} dim={dim} m={m} distinct={distinct}")
+    rng = np.random.default_rng(ns)
+    x = rng.standard_normal((distinct, dim)).astype(np.float32)[rng.integers(0, distinct, ns)]
+    a = rng.integers(0, 3, ns).astype(np.int32)
+    cent = np.repeat(rng.standard_normal((1, dim)).astype(np.float32), 3, axis=0)
+    cb = fg.pq_train(torch.from_numpy(x).cuda(), torch.from_numpy(a).cuda(), torch.from_numpy(cent).cuda(), m,
+                     sample_size=ns, iters=3)
+    assert np.array_equal(_bits(_host(cb)), _bits(oracle.pq_train(x, a, cent, m, sample_size=ns, iters=3)))
+
+
 @pytest.mark.parametrize("n,nlist,distinct", [(256, 1, 256), (2048, 7, 2048), (2049, 300, 40), (6145, 33, 6145)])
 def test_build_lists_at_chunk_edges(n, nlist, distinct):
     """The inverted lists at the edges of the 2048-row chunks they are sorted in: one list, a chunk of one row,
