@@ -485,6 +485,23 @@ def test_pq_train_at_step_edges(ns, dim, m, distinct):
     assert np.array_equal(_bits(_host(cb)), _bits(oracle.pq_train(x, a, cent, m, sample_size=ns, iters=3)))
 
 
+@pytest.mark.parametrize("n,dim,m", [(1, 128, 32), (255, 96, 16), (2049, 96, 32), (4097, 128, 8), (77, 128, 128)])
+def test_pq_encode_ties_and_extremes(n, dim, m):
+    """The nearest codeword of odd row counts when codewords repeat (inside a block of 16 and across blocks: the
+    first wins) and when no distance is below FLT_MAX (overflow, NaN: codeword 0)."""
+    _say(f"pq_encode n={n} dim={dim} m={m}")
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    x[::5] = np.float32(3e30)
+    x[3::7] = np.nan
+    a = rng.integers(0, 4, n).astype(np.int32)
+    cent = rng.standard_normal((4, dim)).astype(np.float32)
+    cb = rng.standard_normal((m, 256, dim // m)).astype(np.float32)
+    cb = cb[:, rng.integers(0, 40, 256)]
+    got = fg.pq_encode(*(torch.from_numpy(v).cuda() for v in (x, a, cent, cb)))
+    assert np.array_equal(_host(got), oracle.pq_encode(x, a, cent, cb, fma_mode=1))
+
+
 @pytest.mark.parametrize("n,nlist,distinct", [(256, 1, 256), (2048, 7, 2048), (2049, 300, 40), (6145, 33, 6145)])
 def test_build_lists_at_chunk_edges(n, nlist, distinct):
     """The inverted lists at the edges of the 2048-row chunks they are sorted in: one list, a chunk of one row,
