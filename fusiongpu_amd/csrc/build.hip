@@ -631,7 +631,10 @@ __global__ __launch_bounds__(kPPBlock) void pp_update_kernel(const float* __rest
 // same chain, on c - x).  The rows read bound it: of 500k rows of 128 dims in
 // 1000 clusters a pass computes a third on average, 14.9 us, 10.4 us in the
 // median.  (One lane a row, 1024 threads and 128 registers of row: 15.0 us; 512
-// threads with half the hand-over buffer a wave: 15.6 us.)
+// threads with half the hand-over buffer a wave: 15.6 us.)  Two lines a load batch:
+// seeding 1M x 128, 1024 centres, 39.3 -> 37.4 ms, 500k 22.9 -> 22.8; four lines
+// 39.3 and 23.4.  (Ruling rows out on a half-size fp16 copy first: 25 and 39 ms, the
+// second look's latency costs what the bytes save.)
 constexpr int kPPThreads = 256;
 template <int D>
 __global__ __launch_bounds__(kPPThreads) void pp_update_rows_kernel(
@@ -667,7 +670,7 @@ __global__ __launch_bounds__(kPPThreads) void pp_update_rows_kernel(
   }
   wave_lds_order();
   for (int p = 0; p < m; p += kWave)
-    dist[p + lane] = wave_rows_l2<D, kWave, 1>(x, list[min(p + lane, m - 1)], cs, tr_s[wave]);
+    dist[p + lane] = wave_rows_l2<D, kWave, 2>(x, list[min(p + lane, m - 1)], cs, tr_s[wave]);
   wave_lds_order();
   uint64_t sum = 0;
 #pragma unroll
