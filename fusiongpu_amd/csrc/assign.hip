@@ -35,8 +35,8 @@
 // so its key is at most
 //     f_m (1 + 2^-16) + 2.001 (g sqrt(D_m) + hn) + 2^-15 D_m,
 // with sqrt(D_m) <= sqrt(Y) + g, Y = f_m (1 + 2^-16) - (bias - 2 E_a X / u - hn).
-// Rows or centroids outside the scales (or not finite) get a NaN bound, which
-// makes every column a candidate.
+// Rows or centroids outside the scales (norms_in_range; or not finite) get a NaN
+// bound, which makes every column a candidate.
 //
 // Candidates.  A lane sees the columns of one class (column mod 32) and keeps
 // the class's smallest key, whose low bits name the tile, and its second
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(kAWaves * kWave, 2) void assign_kernel(const float*
     for (int k = 0; k < 2 * NC; ++k) n2 += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
     n2 += __shfl_xor(n2, 32, kWave);
     const int sx = 13 - max(norm_exp(n2), ce) - sc;  // X^2 / u and u C^2 below 2^13
-    const bool ok = n2 < 0x1p100f && cm < 0x1p100f && sx - sc >= -14 && sx - sc <= 15 && sx >= -126 && sx <= 126;
+    const bool ok = norms_in_range(n2, cm) && sx - sc >= -14 && sx - sc <= 15 && sx >= -126 && sx <= 126;
     const float f = ok ? ldexpf(1.0f, sx) : 0.0f;
     float e2 = 0.0f;
 #pragma unroll

@@ -85,6 +85,20 @@ __device__ __forceinline__ void split3(double v, uint16_t& b1, uint16_t& b2, uin
 __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) { return (uint32_t)lo | ((uint32_t)hi << 16); }
 
 // ---- scales of rows and columns (assign.hip, knn.hip) -----------------------------
+// The margins take the exact fp32 chain as within a relative gamma(130) of the
+// distance.  Near the subnormal range its roundings are absolute, 130 of at most
+// 2^-150: below 2^-142.  Scaled (by at most 2^13 / M, M = max(||x||^2, ||c||^2))
+// that stays below 2^-38 for M >= kNormMin, nothing against the margins' absolute
+// 2^-13; the fp32 norms and rounding errors, whose squares may each have lost
+// 2^-150, keep their bounds too.  Smaller data takes every exact distance: without
+// the limit, of 32768 Gaussian rows of 128 dims 1 lost its nearest of 200 columns
+// at coordinates of 2^-72 and 2542 at 2^-74.
+constexpr float kNormMin = 0x1p-90f;
+constexpr float kNormMax = 0x1p100f;
+// Whether a row of squared norm n2 against columns of at most cn_max has scales.
+__device__ __forceinline__ bool norms_in_range(float n2, float cn_max) {
+  return n2 < kNormMax && cn_max < kNormMax && fmaxf(n2, cn_max) >= kNormMin;
+}
 // n2 < 2^norm_exp(n2), the least such power.
 __device__ __forceinline__ int norm_exp(float n2) {
   int e = 0;

@@ -22,7 +22,8 @@
 //   4. The last lists (about 1.5 k entries) get exact distances; the k smallest
 //      (distance, row) keys are the answer.
 //   5. A query whose list overflows (many tied rows, or a margin as wide as the
-//      distances) or whose norm is out of the scales gets every exact distance.
+//      distances) or whose norm is out of the scales (norms_in_range) gets every exact
+//      distance.
 //
 // The estimate and its margin are assign.hip's, with the query as the row and
 // bias 0: f = D + kappa + e, D the distance scaled by 2^(sx + sc), kappa one
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(64) void knn_query_kernel(const float* __restrict__
   for (int k = 0; k < 2 * NC; ++k) n2 += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
   n2 += __shfl_xor(n2, 32, kWave);
   const int sx = 13 - max(norm_exp(n2), norm_exp(cm)) - sc;  // X^2 / u and u C^2 below 2^13
-  const bool ok = q < nq && n2 < 0x1p100f && cm < 0x1p100f && sx - sc >= -14 && sx - sc <= 15 && sx >= -126 && sx <= 126;
+  const bool ok = q < nq && norms_in_range(n2, cm) && sx - sc >= -14 && sx - sc <= 15 && sx >= -126 && sx <= 126;
   const float f = ok ? ldexpf(1.0f, sx) : 0.0f;
   float e2 = 0.0f;
   uint4* b = ablk + (size_t)blockIdx.x * (NC + 1) * kWave + lane;

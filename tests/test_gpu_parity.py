@@ -163,6 +163,23 @@ def test_l2_topk_nearest_extremes(case):
     assert np.array_equal(_host(ids).view(np.uint32), oid) and np.array_equal(_bits(_host(d)), _bits(od))
 
 
+@pytest.mark.parametrize("dim,e", [(128, -44), (128, -46), (128, -60), (128, -73), (96, -74), (32, -72), (64, -76)])
+def test_l2_topk_nearest_near_subnormal_distances(dim, e):
+    """p = 1 from 32768 rows on, at coordinates of 2^e: around 2^-45, where the margins stop applying, and where
+    squared differences are subnormal and the exact chain rounds in steps of 2^-149.  Some rows are far larger, so
+    that they have a margin against columns that would have none."""
+    _say(f"l2_topk nearest subnormal dim={dim} e={e}")
+    rng = np.random.default_rng(dim - e)
+    x = (rng.standard_normal((32768, dim)) * 2.0**e).astype(np.float32)
+    c = (rng.standard_normal((200, dim)) * 2.0**e).astype(np.float32)
+    x[100:400] *= np.float32(2.0**3)
+    x[400:500] *= np.float32(2.0**20)
+    x[500:510] = 0
+    ids, d = fg.l2_topk(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), 1)
+    oid, od = oracle.coarse(x, c, 1, prune_ratio=np.inf)
+    assert np.array_equal(_bits(_host(d)), _bits(od)) and np.array_equal(_host(ids).view(np.uint32), oid)
+
+
 # --------------------------------------------------------------------------- coarse quantizer (A2, A3)
 @pytest.mark.parametrize("case", ["unit", "x300", "sift_like"])
 def test_coarse_margin_stays_tight_at_large_norms(case):

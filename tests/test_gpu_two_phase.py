@@ -481,6 +481,22 @@ def test_knn_exact_large_base_hand_over(case):
         assert np.array_equal(gid[:24], oid) and np.array_equal(_bits(gd[:24]), _bits(od))
 
 
+@pytest.mark.parametrize("dim,e", [(128, -44), (128, -46), (128, -60), (128, -73), (96, -74), (32, -72), (64, -76)])
+def test_knn_exact_near_subnormal_distances(dim, e):
+    """The large-base pass at coordinates of 2^e: around 2^-45, where the bounds stop applying (a query below it takes
+    every exact distance), and where squared differences are subnormal.  Some queries are far larger than the rows."""
+    _say(f"knn_exact subnormal dim={dim} e={e}")
+    rng = np.random.default_rng(dim - e)
+    x = (rng.standard_normal((20000, dim)) * 2.0**e).astype(np.float32)
+    q = (rng.standard_normal((70, dim)) * 2.0**e).astype(np.float32)
+    q[40:50] *= np.float32(2.0**3)
+    q[50:60] *= np.float32(2.0**20)
+    q[60] = 0
+    gid, gd = fg.knn_exact(torch.from_numpy(q).cuda(), torch.from_numpy(x).cuda(), 10)
+    oid, od = oracle.knn_exact(q, x, 10)
+    assert np.array_equal(_bits(_host(gd)), _bits(od)) and np.array_equal(_host(gid), oid)
+
+
 def test_reference_default_rerank_m_end_to_end():
     """The reference's default rerank_m = 10000 (defs.h:18) through the
     two-phase scan and the exact rerank, against the oracle."""
