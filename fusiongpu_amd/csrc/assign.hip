@@ -36,7 +36,7 @@
 //     f_m (1 + 2^-16) + 2.001 (g sqrt(D_m) + hn) + 2^-15 D_m,
 // with sqrt(D_m) <= sqrt(Y) + g, Y = f_m (1 + 2^-16) - (bias - 2 E_a X / u - hn).
 // Rows or centroids outside the scales (norms_in_range; or not finite) get a NaN
-// bound, which makes every column a candidate.
+// bound, which makes every column a candidate, and rows that are not finite -inf.
 //
 // Candidates.  A lane sees the columns of one class (column mod 32) and keeps
 // the class's smallest key, whose low bits name the tile, and its second
@@ -238,9 +238,10 @@ __global__ __launch_bounds__(kAWaves * kWave, 2) void assign_kernel(const float*
     A[s][NC] = __builtin_bit_cast(f16x8, h ? make_uint4(0u, 0u, 0u, 0u)
                                            : make_uint4(pack2(ub, ub), pack2(ub, kHOne), pack2(k1, k2), pack2(k3, 0u)));
     if (h == 0) {
-      g_s[wave][32 * s + li] = ok ? g : __builtin_nanf("");
+      // f is 0 if not ok, and e2 then 0, or NaN if the row is not finite: no column is its nearest
+      g_s[wave][32 * s + li] = ok ? g : e2 == 0.0f ? __builtin_nanf("") : 0.0f;
       q_s[wave][32 * s + li] = bias - shift - hn;
-      h_s[wave][32 * s + li] = hn;
+      h_s[wave][32 * s + li] = ok ? hn : -INFINITY;
     }
   }
 
@@ -339,7 +340,10 @@ __device__ __forceinline__ float wave_pairs_l2(const float* __restrict__ x, cons
 
 // The candidates' exact distances: a wave takes 64 rows, packs their candidate
 // columns 64 at a time and keeps each row's smallest (distance, column) key.
+// A row all of whose distances overflow has its first column, at distance inf; one
+// that is not finite itself (no candidates) has none (kPadKey).
 constexpr int kRWaves = 4;
+constexpr uint64_t kNoKey = ((uint64_t)0x7F800000u << 32) | (uint32_t)kPadId;  // above every key that is not NaN
 template <int D>
 __global__ __launch_bounds__(kRWaves * kWave, 4) void assign_rescore_kernel(
     const float* __restrict__ x, int64_t n, const float* __restrict__ c, int nc, const uint16_t* __restrict__ cand,
@@ -355,7 +359,7 @@ __global__ __launch_bounds__(kRWaves * kWave, 4) void assign_rescore_kernel(
   uint32_t* q = q_s[wave];  // row << 16 | column
   const int64_t row = row0 + lane;
   const int ncand = row < n ? (int)cnt[row] : 0;
-  best[lane] = kPadKey;
+  best[lane] = kNoKey;
   int nq = 0;
   auto score = [&](int m) {
     wave_lds_order();
@@ -396,7 +400,7 @@ __global__ __launch_bounds__(kRWaves * kWave, 4) void assign_rescore_kernel(
   }
   if (nq > 0) score(nq);
   if (row < n) {
-    const uint64_t k = best[lane];
+    const uint64_t b = best[lane], k = b == kNoKey ? kPadKey : b;
     ids[row] = key_id(k);
     dist[row] = key_dist(k);
   }

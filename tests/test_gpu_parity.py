@@ -163,6 +163,27 @@ def test_l2_topk_nearest_extremes(case):
     assert np.array_equal(_host(ids).view(np.uint32), oid) and np.array_equal(_bits(_host(d)), _bits(od))
 
 
+@pytest.mark.parametrize("dim,nc", [(128, 64), (96, 1024), (32, 100)])
+def test_l2_topk_nearest_overflowing_distances(dim, nc):
+    """Finite rows whose squared distances overflow, to every column (the first one then, at distance inf) or to all but
+    a few equally large ones, beside ordinary rows."""
+    _say(f"l2_topk nearest overflow dim={dim} nc={nc}")
+    rng = np.random.default_rng(dim + nc)
+    x = rng.standard_normal((32768, dim)).astype(np.float32)
+    c = rng.standard_normal((nc, dim)).astype(np.float32)
+    x[100:150] *= np.float32(1e20)
+    x[150:200] = np.float32(3e38)
+
+    def check():
+        ids, d = fg.l2_topk(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), 1)
+        oid, od = oracle.coarse(x, c, 1, prune_ratio=np.inf)
+        assert np.array_equal(_host(ids), oracle.kmeans_assign(x, c)[:, None])
+        assert np.array_equal(_bits(_host(d)), _bits(od))
+    check()
+    c[nc - 2], c[nc - 1] = x[120], x[160]
+    check()
+
+
 @pytest.mark.parametrize("dim,e", [(128, -44), (128, -46), (128, -60), (128, -73), (96, -74), (32, -72), (64, -76)])
 def test_l2_topk_nearest_near_subnormal_distances(dim, e):
     """p = 1 from 32768 rows on, at coordinates of 2^e: around 2^-45, where the margins stop applying, and where
