@@ -53,6 +53,11 @@ std::vector<int32_t> assign(const float* d_x, int64_t n, const float* d_c, int k
   ok(fgpu_l2_topk(d_x, n, d_c, k, dim, 1, a.p, d.p, ws.p, wb, nullptr), "assignment");
   std::vector<int32_t> h(n);
   hip_ok(hipMemcpy(h.data(), a.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost), "copy assignment");
+  for (int64_t i = 0; i < n; ++i)
+    if (h[i] < 0 || h[i] >= k) {
+      std::fprintf(stderr, "row %lld has no finite distance to a centroid\n", (long long)i);
+      std::exit(1);
+    }
   return h;
 }
 

@@ -209,13 +209,14 @@ __global__ __launch_bounds__(256) void order_sum_kernel(const float* __restrict_
 }
 
 __global__ __launch_bounds__(256) void kmeans_accumulate_kernel(
-    const float* __restrict__ x, int64_t n, const int32_t* __restrict__ assign, int dim, int shift,
+    const float* __restrict__ x, int64_t n, const int32_t* __restrict__ assign, int k, int dim, int shift,
     unsigned long long* __restrict__ sums, int32_t* __restrict__ counts) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n * dim) return;
   const int64_t i = t / dim;
   const int d = (int)(t % dim);
   const int c = assign[i];
+  if ((uint32_t)c >= (uint32_t)k) return;  // a row without a centre (no finite distance)
   const long long q = __float2ll_rn(ldexpf(x[t], shift));
   atomicAdd(&sums[(int64_t)c * dim + d], (unsigned long long)q);
   if (d == 0) atomicAdd(&counts[c], 1);
@@ -941,7 +942,7 @@ fgpu_status launch_kmeans_accumulate(const float* x, int64_t n, const int32_t* a
   const size_t fixed = order_fixed_bytes(k);
   const int64_t fit = ows && ows_bytes > fixed ? (int64_t)((ows_bytes - fixed) / sizeof(int32_t)) : 0;
   if (n < kOrderedMinRows || k > kOrderedMaxCentres || dim > 256 || fit < std::min<int64_t>(n, kOrderedMinRows))
-    return launch1d(kmeans_accumulate_kernel, n * dim, 256, s, x, n, assign, dim, shift, sums, counts);
+    return launch1d(kmeans_accumulate_kernel, n * dim, 256, s, x, n, assign, k, dim, shift, sums, counts);
   Carve cv(ows, ows_bytes);
   int32_t* cursor = cv.take<int32_t>((size_t)k + 1);
   int32_t* cnt = cv.take<int32_t>((size_t)k);  // this chunk's counts

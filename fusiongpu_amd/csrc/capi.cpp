@@ -1521,9 +1521,6 @@ fgpu_status fgpu_build_ivfpq_sampled(const float* dx, int64_t n, int dim, int nl
     FGPU_TRY(fgpu_l2_topk(dx, n, cent.p, nlist, dim, 1, assign.p, dist.p, tws.p, tb, stream));
     FGPU_HIP(hipStreamSynchronize(s));
   }
-  FGPU_CHECK(pq_ok && pq_iters >= 0, FGPU_ERR_ARG, "build: pq_m must divide dim, pq_iters >= 0 and 256 sample rows or more");
-  FGPU_TRY(pq_train_sampled(dx, dim, pq_m, assign.p, cent.p, sample.valid() ? sample.get() : PqSample(n, pq_m, sample_size),
-                            pq_iters, cb.p, s));
   // inverted lists in cluster order, ids ascending inside a list
   // (build_global.cu:225-240); the codes are written in that order
   DevBuf<int32_t> offs, ids, pos;
@@ -1534,6 +1531,15 @@ fgpu_status fgpu_build_ivfpq_sampled(const float* dx, int64_t n, int dim, int nl
   FGPU_TRY(pos.alloc(n));
   FGPU_TRY(lws.alloc(lb));
   FGPU_TRY(launch_list_order(assign.p, n, nlist, offs.p, ids.p, pos.p, lws.p, lb, s));
+  // A row without a finite distance to any centroid (NaN, or an overflow) has no
+  // list: PQ training and encoding would read past the centroids for it.
+  int32_t listed = 0;
+  FGPU_HIP(hipMemcpyAsync(&listed, offs.p + nlist, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  FGPU_HIP(hipStreamSynchronize(s));
+  FGPU_CHECK(listed == n, FGPU_ERR_ARG, "build: " + std::to_string(n - listed) + " rows have no finite distance to a centroid");
+  FGPU_CHECK(pq_ok && pq_iters >= 0, FGPU_ERR_ARG, "build: pq_m must divide dim, pq_iters >= 0 and 256 sample rows or more");
+  FGPU_TRY(pq_train_sampled(dx, dim, pq_m, assign.p, cent.p, sample.valid() ? sample.get() : PqSample(n, pq_m, sample_size),
+                            pq_iters, cb.p, s));
   FGPU_TRY(launch_pq_encode(dx, n, dim, pq_m, assign.p, cent.p, cb.p, codes.p, s, 1, pos.p));
   FGPU_HIP(hipMemcpyAsync(h_offsets, offs.p, sizeof(int32_t) * ((size_t)nlist + 1), hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipMemcpyAsync(h_ids, ids.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost, s));

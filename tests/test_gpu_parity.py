@@ -427,6 +427,23 @@ def test_kmeans_update_grouped_rows(n, k, dim, chunk):
     assert np.array_equal(_bits(_host(c)), _bits(want))
 
 
+@pytest.mark.parametrize("n", [2000, 40000])
+def test_kmeans_update_skips_rows_without_a_centre(n):
+    """Rows whose assignment is out of range (a row without a finite distance gets INT_MAX) count for no centre, in
+    the form with one atomic a coordinate and in the grouped one."""
+    _say(f"kmeans_update rows without a centre n={n}")
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, 32)).astype(np.float32)
+    a = rng.integers(0, 9, n).astype(np.int32)
+    out = rng.random(n) < 0.1
+    out[-1] = True
+    bad = np.where(out, rng.choice([np.iinfo(np.int32).max, -1, 9], n), a).astype(np.int32)
+    c = torch.zeros(9, 32, device="cuda")
+    cnt = fg.kmeans_update(torch.from_numpy(x).cuda(), torch.from_numpy(bad).cuda(), c, 30, 0)
+    want, wcnt = oracle.kmeans_update(x[~out], a[~out], np.zeros((9, 32), np.float32), 30, 0)
+    assert np.array_equal(_host(cnt), wcnt) and np.array_equal(_bits(_host(c)), _bits(want))
+
+
 @pytest.mark.parametrize("shift", [48, 0, 60])
 def test_kmeans_update_rounds_like_the_oracle(shift):
     """round(x 2^shift) of every magnitude: halves (ties to even), around 2^50, where the grouped form's conversion
@@ -571,6 +588,18 @@ def test_build_lists_at_chunk_edges(n, nlist, distinct):
     want = oracle.build_ivfpq(x, nlist, 16, **kw)
     for g, w, name in zip(got, want, ["offsets", "ids", "codes", "centroids", "codebook"]):
         assert np.array_equal(np.asarray(g).view(np.uint8), np.asarray(w).view(np.uint8)), name
+
+
+@pytest.mark.parametrize("n,train_rows,value", [(3000, 0, np.nan), (40000, 0, np.nan), (3000, 1000, np.inf)])
+def test_build_refuses_rows_without_a_list(n, train_rows, value):
+    """A row with no finite distance to any centroid has no list; the build returns an error before its PQ training."""
+    _say(f"build refuses n={n} train_rows={train_rows} value={value}")
+    x = oracle.gen_gmm(n, 32, 8, seed=n, sig_lo=0.1)
+    x[n // 2 + 1, 5] = value
+    kw = dict(train_rows=train_rows) if train_rows else {}
+    with pytest.raises(RuntimeError, match="1 rows have no finite distance"):
+        fg.build_ivfpq(torch.from_numpy(x).cuda(), 40, 16, kmeans_iters=2, init_mode=0, seed=3, pq_iters=1,
+                       sample_size=256, **kw)
 
 
 def test_config1_end_to_end_bit_exact():
