@@ -225,6 +225,11 @@ bool screen_pays(const fgpu_index* ix, int nq, int k, bool flow) {
   return !flow || ix->total < kScreenAnyBatch || nq > (k > 32 ? kFlowWideK : kFlowRound);
 }
 
+// fgpu_search's words after the probe arrays: the flow kernel's query counter and
+// the route of the call, whether the workspace holds the screen's counters.
+constexpr int kSearchWords = 2;
+constexpr int kRouteLut = 1, kRouteCounters = 2;
+
 // The screen's workspace, carved from `base` (fgpu_search, after the probe
 // arrays).  The counters, per-list counts and per-query candidate counts are
 // one contiguous block that the first screen kernel zeroes.
@@ -687,7 +692,7 @@ fgpu_status fgpu_row_gather(const void* d_rows, int64_t nrows, int row_bytes, co
 namespace fgpu {
 size_t search_lut_workspace_bytes(int nq, int nlist, int nprobe) {
   return carve_bytes<uint32_t>((size_t)nq * nprobe) + carve_bytes<float>((size_t)nq * nprobe) +
-         carve_bytes<int>(1) + fgpu_coarse_workspace_bytes(nq, nlist);
+         carve_bytes<int>(kSearchWords) + fgpu_coarse_workspace_bytes(nq, nlist);
 }
 }  // namespace fgpu
 
@@ -700,7 +705,7 @@ size_t fgpu_search_workspace_bytes(int nq, int nlist, int nprobe) {
   const size_t coarse = fgpu_coarse_workspace_bytes(nq, nlist);
   // (A small batch's select sets up the scan's words while it reads the tile.)
   return carve_bytes<uint32_t>((size_t)nq * nprobe) + carve_bytes<float>((size_t)nq * nprobe) +
-         carve_bytes<int>(1) + (nq <= kSmallBatch ? coarse + screen : std::max(coarse, screen));
+         carve_bytes<int>(kSearchWords) + (nq <= kSmallBatch ? coarse + screen : std::max(coarse, screen));
 }
 
 fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprobe, int k, float prune_ratio,
@@ -709,7 +714,7 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   Carve cv(ws, ws_bytes);
   uint32_t* pid = cv.take<uint32_t>((size_t)nq * nprobe);
   float* pd = cv.take<float>((size_t)nq * nprobe);
-  int* qctr = cv.take<int>(1);
+  int* qctr = cv.take<int>(kSearchWords);
   FGPU_CHECK(cv.ok(), FGPU_ERR_WORKSPACE, "search: workspace too small");
   FGPU_CHECK(nq >= 0 && k >= 1, FGPU_ERR_ARG, "search: bad sizes");
   FGPU_CHECK(adc_supported(ix->dim, ix->m), FGPU_ERR_UNSUPPORTED, "search: no kernel for this (dim, pq_m)");
@@ -743,6 +748,8 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
     a.qlist = nullptr;
     a.hand_thr = sw.thr;
     SelectSide side;
+    side.ctr = qctr;
+    side.route = kRouteCounters;
     side.zero = sw.zero;
     side.nzero = (int)ScreenWs::zero_words(nq, ix->nlist);
     side.flag_at = kCtrFlag;
@@ -759,7 +766,10 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   if (ix->screen_ok && ix->opt_screen && k <= 64 && nq > 0 && screen_pays(ix, nq, k, flow) && ((uintptr_t)dq & 15) == 0 &&
       ix->nlist <= kScreenMaxLists && (int64_t)nq * nprobe < INT32_MAX &&
       sw.carve(rest, rest_bytes, nq, ix->nlist, nprobe)) {
-    FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream, {}));
+    SelectSide side;
+    side.ctr = qctr;
+    side.route = kRouteCounters;
+    FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream, side));
     FGPU_HIP(mark(1));
     ScreenArgs sa{dq, ix->d_centroids, ix->d_offsets, ix->d_codes, ix->d_ids, ix->d_codebook, ix->d_cb16,
                   ix->d_vext, ix->d_rmax, pid, pd, nq, nprobe, k, ix->nlist};
@@ -791,8 +801,9 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   // coarse step's select stores that value on the way.
   const int grid = flow_grid(ix->dim, ix->m, nq, nprobe);
   SelectSide side;
-  side.ctr = grid > 0 ? qctr : nullptr;
+  side.ctr = qctr;
   side.ctr_val = grid;
+  side.route = kRouteLut;
   FGPU_TRY(coarse_search(ix, dq, nq, nprobe, prune_ratio, pid, pd, rest, rest_bytes, stream, side));
   for (int i = 1; i < kStageEvents - 1; ++i) FGPU_HIP(mark(i));  // no screen stages
   AdcArgs a = adc_args(ix, dq, nq, pid, pd, nprobe, k, d_out_ids, d_out_dists);
@@ -820,12 +831,20 @@ fgpu_status fgpu_search_screen_stats(const fgpu_index* ix, int nq, int nprobe, c
   Carve cv(const_cast<void*>(ws), ws_bytes);
   cv.take<uint32_t>((size_t)nq * nprobe);
   cv.take<float>((size_t)nq * nprobe);
-  cv.take<int>(1);
+  const int* words = cv.take<int>(kSearchWords);
   FGPU_CHECK(cv.ok(), FGPU_ERR_WORKSPACE, "search_screen_stats: workspace too small");
   ScreenWs sw;
   FGPU_CHECK(sw.carve(cv.base + cv.used, ws_bytes - cv.used, nq, ix->nlist, nprobe), FGPU_ERR_WORKSPACE,
              "search_screen_stats: workspace too small for the screen");
   hipStream_t s = as_stream(stream);
+  // Without counters the screen's words hold what the coarse step left there.
+  int route[kSearchWords];
+  FGPU_HIP(hipMemcpyAsync(route, words, sizeof(route), hipMemcpyDeviceToHost, s));
+  FGPU_HIP(hipStreamSynchronize(s));
+  if (route[1] != kRouteCounters) {
+    for (int i = 0; i < n_stats; ++i) h_stats[i] = i == 5 && route[1] == kRouteLut ? nq : 0;
+    return FGPU_OK;
+  }
   std::vector<int> z(ScreenWs::zero_words(nq, ix->nlist));
   std::vector<float> thr((size_t)nq);
   FGPU_HIP(hipMemcpyAsync(z.data(), sw.zero, sizeof(int) * z.size(), hipMemcpyDeviceToHost, s));

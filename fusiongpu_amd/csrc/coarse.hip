@@ -640,7 +640,10 @@ __device__ __forceinline__ void select_row(const float (&val)[VPL], int64_t row,
 // The launch's side words, by its first workgroup.
 __device__ __forceinline__ void side_words(const SelectSide& s, int64_t nrows) {
   if (blockIdx.x != 0) return;
-  if (s.ctr && threadIdx.x == 0) *s.ctr = s.ctr_val;
+  if (s.ctr && threadIdx.x == 0) {
+    s.ctr[0] = s.ctr_val;
+    s.ctr[1] = s.route;
+  }
   if (s.zero)
     for (int i = threadIdx.x; i < s.nzero; i += blockDim.x) s.zero[i] = i == s.flag_at ? s.flag : 0;
   if (s.hand)

@@ -27,12 +27,13 @@ fgpu_status launch_gemm_est(const float* x, int64_t nrows, const float* c, int n
 fgpu_status launch_gemm_est_sel(const float* x, int64_t nrows, const float* c, int ncols, int dim, const float* cn,
                                 const float* cn_max, void* est, int64_t ld, hipStream_t s);
 int64_t est_sel_ld(int ncols);
-// Words the coarse select stores for the kernels after it: *ctr = ctr_val (the
-// flow scan's query counter); zero[0 .. nzero) = 0 except zero[flag_at] = flag;
+// Words the coarse select stores for the kernels after it: ctr[0] = ctr_val (the
+// flow scan's query counter) and ctr[1] = route (what fgpu_search_screen_stats
+// finds); zero[0 .. nzero) = 0 except zero[flag_at] = flag;
 // each row's hand[row stride .. + 2] = kPadKey and 0 (AdcArgs::hand).
 struct SelectSide {
   int* ctr = nullptr;
-  int ctr_val = 0;
+  int ctr_val = 0, route = 0;
   int* zero = nullptr;
   int nzero = 0, flag_at = 0, flag = 0;
   uint32_t* hand = nullptr;

@@ -206,8 +206,9 @@ fgpu_status fgpu_search(const fgpu_index* idx, const float* d_queries, int nq, i
  * probes: no usable probe, or one probe holding fewer than k vectors), 0;
  * h_stats[8..15] the clocks of FGPU_OPT_SCREEN_CLOCKS;
  * h_stats[16..19] = (query, vector) pairs screened in round 1 and round 2,
- * MFMA tiles (32 queries x 32 vectors) run in round 1 and round 2.  Only
- * meaningful after a call that took the screen. */
+ * MFMA tiles (32 queries x 32 vectors) run in round 1 and round 2.  A call
+ * that the LUT kernels answered alone counts its nq queries in h_stats[5] (and
+ * none screened: h_stats[0..4] = 0). */
 fgpu_status fgpu_search_screen_stats(const fgpu_index* idx, int nq, int nprobe, const void* d_workspace,
                                      size_t workspace_bytes, void* stream, long long* h_stats, int n_stats);
 /* 1 when the index carries the screen's arrays (built at creation for the

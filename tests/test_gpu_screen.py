@@ -445,3 +445,30 @@ def test_search_route_edges(dim, m, nq, k):
     q = fg.gen_gmm(nq, dim, 32, seed=dim + m, set=1, sig_lo=0.08)
     _check(idx, q, cent, cb, offs, ids, codes, 70 if nq == 767 else 10, k, screened=False)
     idx.close()
+
+
+@pytest.mark.parametrize("dim,m,nq,nprobe,k,screened", [(128, 32, 200, 8, 10, False), (128, 32, 257, 8, 10, True),
+                                                        (96, 32, 100, 8, 10, False), (128, 32, 600, 8, 40, False),
+                                                        (128, 32, 20, 8, 10, False), (128, 32, 300, 8, 64, False)])
+def test_screen_counters_follow_the_route(dim, m, nq, nprobe, k, screened):
+    """fgpu_search_screen_stats after a search that the LUT kernels answered (an index of 66,000 vectors): every query
+    counted there and nothing screened, also where the workspace held a screened search before; and with the screen
+    off."""
+    _say(f"screen counters dim={dim} m={m} nq={nq} k={k}")
+    offs, ids, codes, cent, cb = _gmm_index(dim, m, 128, 66000, seed=dim + m)
+    idx = fg.Index.from_arrays(dim, m, offs, ids, codes, cent, cb)
+    q = torch.from_numpy(fg.gen_gmm(nq, dim, 32, seed=dim + m, set=1, sig_lo=0.08)).cuda()
+    ws = torch.full((idx.search_workspace_bytes(nq, nprobe),), 0x55, dtype=torch.uint8, device="cuda")
+    work = ("pairs_round1", "lists_round2", "pairs_round2", "candidates", "max_candidates", "vector_pairs_round1",
+            "tiles_round1", "tiles_round2")
+    idx.search(q, nprobe, k, workspace=ws)
+    st = idx.search_screen_stats(nq, nprobe, ws)
+    if screened:
+        assert st["pairs_round1"] > 0 and st["candidates"] >= nq * k and st["queries_to_lut_kernel"] <= nq
+    else:
+        assert st["queries_to_lut_kernel"] == nq and not any(st[w] for w in work)
+    idx.set_option(fg.Index.OPT_SCREEN, 0)
+    idx.search(q, nprobe, k, workspace=ws)
+    st = idx.search_screen_stats(nq, nprobe, ws)
+    assert st["queries_to_lut_kernel"] == nq and not any(st[w] for w in work)
+    idx.close()
