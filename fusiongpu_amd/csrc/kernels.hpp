@@ -69,7 +69,11 @@ fgpu_status launch_assign(const float* x, int64_t n, const float* c, int nc, int
 // an estimate matrix.  knn_screen_takes: whether it applies (dim 32, 64, 96 or
 // 128, 16-byte aligned arrays, at least kKnnScreenMinRows base rows, a workspace
 // of about knn_screen_ws_bytes) rather than launch_gemm_est + launch_knn_chunk.
-constexpr int64_t kKnnScreenMinRows = 16384;
+// Its dozen launches cost what four chunks of 4096 rows do, whatever the number of
+// queries.  Measured (us, chunks / this, 128 dims): 16384 rows 68 / 72 (1 query,
+// k 1), 93 / 104 (1, k 100), 124 / 124 (64, k 100), 136 / 130 (256, k 100); 18432
+// rows 83 / 73, 110 / 105, 143 / 125 and 155 / 131.
+constexpr int64_t kKnnScreenMinRows = 4 * 4096 + 1;
 size_t knn_screen_ws_bytes(int nq, int64_t n);
 bool knn_screen_takes(const float* x, int nq, const float* c, int64_t n, int dim, size_t ws_bytes);
 fgpu_status launch_knn_screen(const float* x, int nq, const float* c, int64_t n, int dim, int k, void* ws,

@@ -414,10 +414,13 @@ fgpu_status fgpu_l2_topk(const float* d_x, int64_t n, const float* d_c, int nc, 
  * L2 in the reference's device form, ascending (distance, row index) -- the
  * reference's strict-< insertion keeps the earlier row on ties; padding -1 /
  * FLT_MAX when n < k.  MFMA estimates with a rigorous error margin pick the
- * rows that are re-scored exactly: for 16384 rows or more of dim 32, 64, 96 or
+ * rows that are re-scored exactly: for more than 16384 rows of dim 32, 64, 96 or
  * 128 (16-byte aligned arrays) against a threshold per query that tightens as
  * the base goes by, otherwise chunk by chunk of 4096 rows.  k <= 128, dim <= 256
- * and a multiple of 4, n < 2^31. */
+ * and a multiple of 4, n < 2^31.  The workspace asked for holds up to 2^20 base
+ * rows as MFMA operands (288 MB) beside 17 KB a query (up to 16384 of them); with
+ * less, down to 32768 rows (9 MB), they go in more launches, and below that the
+ * call goes chunk by chunk (a few MB).  The results are the same. */
 size_t fgpu_knn_exact_workspace_bytes(int nq, int64_t n);
 fgpu_status fgpu_knn_exact(const float* d_queries, int nq, const float* d_base, int64_t n, int dim, int k,
                            int32_t* d_ids, float* d_dists, void* d_workspace, size_t workspace_bytes,
