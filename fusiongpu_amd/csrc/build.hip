@@ -90,8 +90,8 @@ __global__ void gather_rows_kernel(const float* __restrict__ x, int dim, const i
 // atomics): integer addition is associative, so the result does not depend on
 // the order the atomics land, unlike the reference's float atomicAdd
 // (kmeans_gpu.cuh:94-97).
-// Two forms.  kmeans_accumulate_kernel: one 64-bit atomic a coordinate.  From
-// kOrderedMinRows rows on, the rows are first grouped by centre (a histogram, its
+// Two forms.  kmeans_accumulate_kernel: one 64-bit atomic a coordinate.  Where
+// grouping_pays, the rows are first grouped by centre (a histogram, its
 // scan, a scatter of the row numbers; the order within a centre is free), then
 // each wave sums 128 consecutive grouped rows in registers and adds a centre's
 // sums once: 1M rows of 128 dims and 4096 centres 0.90 -> 0.14 ms (128 M
@@ -930,6 +930,20 @@ fgpu_status launch_maxabs(const float* x, int64_t count, float* out, hipStream_t
   return launch_max_reduce(out, 1023, out + 1023, s);
 }
 
+// From kOrderedMinRows rows on, the form that takes less time by these fits (us).
+// Atomics: 7.5 a million of them, at least 24, and 0.22 for each row a centre
+// has on average (they queue on its sums).  Grouped: the launches, a row's loads
+// (64 dims each), and the scan and the histograms of the centres.  Measured,
+// atomics / grouped: 32768 rows of 128 dims, 256 centres 70 / 39, 1024 40 / 41,
+// 4096 35 / 52, 16384 42 / 86; 65536 rows, 4096 60 / 53, 8192 61 / 64; 131072 rows,
+// 16384 115 / 83; 65536 rows of 32 dims, 256 95 / 35, 2048 29 / 39; 262144 rows,
+// 8192 68 / 56, 16384 66 / 71; 32768 rows of 200 dims, 256 80 / 53, 2048 49 / 59.
+static bool grouping_pays(int64_t n, int k, int dim) {
+  const double atomics = std::max(24.0, 7.5 * (double)n * dim / (1 << 20)) + 0.22 * (double)n / k;
+  return n >= kOrderedMinRows && k <= kOrderedMaxCentres && dim <= 256 &&
+         atomics > 28.0 + 8.0 * ((dim + 63) / 64) + 3.75 * k / 1024;
+}
+
 // Grouping scratch: the centres' offsets and chunk counts, and the row order.
 static size_t order_fixed_bytes(int k) { return carve_bytes<int32_t>((size_t)k + 1) + carve_bytes<int32_t>(k) + 256; }
 size_t kmeans_order_bytes(int k, int64_t rows) { return order_fixed_bytes(k) + carve_bytes<int32_t>(rows); }
@@ -941,7 +955,7 @@ fgpu_status launch_kmeans_accumulate(const float* x, int64_t n, const int32_t* a
   FGPU_TRY(launch1d(fill_i32_kernel, (int64_t)k, 256, s, counts, (int64_t)k));
   const size_t fixed = order_fixed_bytes(k);
   const int64_t fit = ows && ows_bytes > fixed ? (int64_t)((ows_bytes - fixed) / sizeof(int32_t)) : 0;
-  if (n < kOrderedMinRows || k > kOrderedMaxCentres || dim > 256 || fit < std::min<int64_t>(n, kOrderedMinRows))
+  if (!grouping_pays(n, k, dim) || fit < std::min<int64_t>(n, kOrderedMinRows))
     return launch1d(kmeans_accumulate_kernel, n * dim, 256, s, x, n, assign, k, dim, shift, sums, counts);
   Carve cv(ows, ows_bytes);
   int32_t* cursor = cv.take<int32_t>((size_t)k + 1);

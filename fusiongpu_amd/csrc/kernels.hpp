@@ -423,9 +423,8 @@ fgpu_status launch_probe_counts(const uint32_t* probes, int nq, int nprobe, int 
 fgpu_status launch_maxabs(const float* x, int64_t count, float* out, hipStream_t s);
 // sums and counts of the rows of each centre; ows (may be null): scratch of
 // kmeans_order_bytes(k, rows), with which kOrderedMinRows rows or more are
-// grouped by centre first, up to `rows` at a time.  Below that the one-atomic-a-
-// coordinate form is as fast; above kOrderedMaxCentres the histogram does not
-// fit LDS.
+// grouped by centre first where that is faster (grouping_pays), up to `rows` at a
+// time.  Above kOrderedMaxCentres the histogram does not fit LDS.
 constexpr int64_t kOrderedMinRows = 32768;
 constexpr int kOrderedMaxCentres = 16384;
 constexpr int64_t kOrderedChunk = 1 << 20;

@@ -427,6 +427,21 @@ def test_kmeans_update_grouped_rows(n, k, dim, chunk):
     assert np.array_equal(_bits(_host(c)), _bits(want))
 
 
+@pytest.mark.parametrize("n,k,dim", [(400000, 16384, 36), (400000, 16385, 36), (65536, 4096, 128), (65536, 8192, 128),
+                                     (60000, 1500, 32), (33000, 1500, 128)])
+def test_kmeans_update_both_sides_of_the_grouping_line(n, k, dim):
+    """Centre counts and sizes on both sides of the line between grouping the rows and one atomic a coordinate,
+    the largest centre count the grouping takes among them."""
+    _say(f"kmeans_update grouping line n={n} k={k} dim={dim}")
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    a = rng.integers(0, k, n).astype(np.int32)
+    c = torch.zeros(k, dim, device="cuda")
+    cnt = fg.kmeans_update(torch.from_numpy(x).cuda(), torch.from_numpy(a).cuda(), c, 30, 0)
+    want, wcnt = oracle.kmeans_update(x, a, np.zeros((k, dim), np.float32), 30, 0)
+    assert np.array_equal(_host(cnt), wcnt) and np.array_equal(_bits(_host(c)), _bits(want))
+
+
 @pytest.mark.parametrize("n", [2000, 40000])
 def test_kmeans_update_skips_rows_without_a_centre(n):
     """Rows whose assignment is out of range (a row without a finite distance gets INT_MAX) count for no centre, in
