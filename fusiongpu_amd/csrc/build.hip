@@ -311,11 +311,11 @@ __device__ __forceinline__ void pq_nearest(const float (&r)[R][S], const float* 
 // (pq_utils.h:160-166, built without FMA): the product and the sum each rounded.
 // A thread takes the same subspace of kPQRows rows; one workgroup a CU, as the
 // codebook fills its LDS, each staging it once.
-// pos (may be null): row i's codes go to row pos[i].
+// pos (may be null): row i's codes go to row pos[i], nowhere if it is below 0.
 template <int S, bool FMA>
 __global__ __launch_bounds__(1024) void pq_encode_kernel(const float* __restrict__ x, int64_t n, int dim, int m,
                                                          const int32_t* __restrict__ assign,
-                                                         const float* __restrict__ cent,
+                                                         const float* __restrict__ cent, uint32_t ncent,
                                                          const float* __restrict__ codebook,
                                                          const int32_t* __restrict__ pos,
                                                          uint8_t* __restrict__ codes) {
@@ -334,7 +334,8 @@ __global__ __launch_bounds__(1024) void pq_encode_kernel(const float* __restrict
     for (int q = 0; q < kPQRows; ++q) {
       const int64_t i = min(i0 + q, n - 1);
       const float* xi = x + i * dim + sub * S;
-      const float* ci = cent + (int64_t)assign[i] * dim + sub * S;
+      const uint32_t c = (uint32_t)assign[i];
+      const float* ci = cent + (int64_t)(c < ncent ? c : 0u) * dim + sub * S;
 #pragma unroll
       for (int j = 0; j < S; ++j) r[q][j] = xi[j] - ci[j];
     }
@@ -342,7 +343,10 @@ __global__ __launch_bounds__(1024) void pq_encode_kernel(const float* __restrict
     pq_nearest<S, FMA, kPQRows>(r, cbs + sub * S, m * S, bk);
 #pragma unroll
     for (int q = 0; q < kPQRows; ++q)
-      if (i0 + q < n) codes[(pos ? (int64_t)pos[i0 + q] : i0 + q) * m + sub] = (uint8_t)bk[q];
+      if (i0 + q < n) {
+        const int64_t to = pos ? (int64_t)pos[i0 + q] : i0 + q;
+        if (to >= 0) codes[to * m + sub] = (uint8_t)bk[q];
+      }
   }
 }
 
@@ -411,6 +415,8 @@ __global__ __launch_bounds__(64) void list_scatter_kernel(const int32_t* __restr
       const int32_t p = offsets[l] + at + before;
       ids[p] = (int32_t)i;
       pos[i] = p;
+    } else if (i < r1) {
+      pos[i] = -1;
     }
   }
 }
@@ -418,12 +424,13 @@ __global__ __launch_bounds__(64) void list_scatter_kernel(const int32_t* __restr
 // ---- A15: PQ codebook training (pq_utils.h:17-138) ------------------------------
 __global__ void pq_residuals_kernel(const float* __restrict__ x, int dim, const int32_t* __restrict__ rows,
                                     int nrows, const int32_t* __restrict__ assign,
-                                    const float* __restrict__ cent, float* __restrict__ res) {
+                                    const float* __restrict__ cent, uint32_t ncent, float* __restrict__ res) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)nrows * dim) return;
   const int r = (int)(t / dim), d = (int)(t % dim);
   const int64_t o = rows[r];
-  res[t] = x[o * dim + d] - cent[(int64_t)assign[o] * dim + d];
+  const uint32_t c = (uint32_t)assign[o];
+  res[t] = x[o * dim + d] - cent[(int64_t)(c < ncent ? c : 0u) * dim + d];
 }
 
 // codebook[m][c][j] = res[init_rows[m][c]][m*S + j]
@@ -1035,7 +1042,8 @@ fgpu_status launch_list_order(const int32_t* assign, int64_t n, int nlist, int32
 }
 
 fgpu_status launch_pq_encode(const float* x, int64_t n, int dim, int m, const int32_t* assign, const float* cent,
-                             const float* codebook, uint8_t* codes, hipStream_t s, int fma_mode, const int32_t* pos) {
+                             const float* codebook, uint8_t* codes, hipStream_t s, int fma_mode, int ncent,
+                             const int32_t* pos) {
   const int S = dim / m;
   const size_t lds = (size_t)kPQK * dim * sizeof(float);
   FGPU_CHECK(lds <= 160 * 1024, FGPU_ERR_UNSUPPORTED, "pq_encode: codebook exceeds LDS");
@@ -1046,8 +1054,8 @@ fgpu_status launch_pq_encode(const float* x, int64_t n, int dim, int m, const in
   if (S == SS && (fma_mode != 0) == F) {                                                                      \
     FGPU_HIP(hipFuncSetAttribute((const void*)pq_encode_kernel<SS, F>, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                  (int)lds));                                                                  \
-    hipLaunchKernelGGL((pq_encode_kernel<SS, F>), dim3(grid), dim3(1024), lds, s, x, n, dim, m, assign, cent, codebook, \
-                       pos, codes);                                                                               \
+    hipLaunchKernelGGL((pq_encode_kernel<SS, F>), dim3(grid), dim3(1024), lds, s, x, n, dim, m, assign, cent, (uint32_t)ncent, \
+                       codebook, pos, codes);                                                                         \
     FGPU_HIP(hipGetLastError());                                                                              \
     return FGPU_OK;                                                                                           \
   }
@@ -1060,8 +1068,9 @@ fgpu_status launch_pq_encode(const float* x, int64_t n, int dim, int m, const in
 }
 
 fgpu_status launch_pq_residuals(const float* x, int dim, const int32_t* rows, int nrows, const int32_t* assign,
-                                const float* cent, float* res, hipStream_t s) {
-  return launch1d(pq_residuals_kernel, (int64_t)nrows * dim, 256, s, x, dim, rows, nrows, assign, cent, res);
+                                const float* cent, int ncent, float* res, hipStream_t s) {
+  return launch1d(pq_residuals_kernel, (int64_t)nrows * dim, 256, s, x, dim, rows, nrows, assign, cent, (uint32_t)ncent,
+                  res);
 }
 
 fgpu_status launch_pq_init(const float* res, int nsample, int dim, int m, const int32_t* init_rows, float* codebook,

@@ -379,7 +379,7 @@ struct PqSample {
 };
 
 fgpu_status pq_train_sampled(const float* dx, int dim, int pq_m, const int32_t* d_assign, const float* d_cent,
-                             const PqSample& sm, int iters, float* d_codebook, hipStream_t s) {
+                             int ncent, const PqSample& sm, int iters, float* d_codebook, hipStream_t s) {
   const int actual = sm.actual;
   DevBuf<int32_t> drows, dinit;
   DevBuf<uint8_t> dassign;
@@ -390,7 +390,7 @@ fgpu_status pq_train_sampled(const float* dx, int dim, int pq_m, const int32_t* 
   FGPU_TRY(res.alloc((size_t)actual * dim));
   FGPU_HIP(hipMemcpyAsync(drows.p, sm.rows.data(), sizeof(int32_t) * actual, hipMemcpyHostToDevice, s));
   FGPU_HIP(hipMemcpyAsync(dinit.p, sm.init.data(), sizeof(int32_t) * sm.init.size(), hipMemcpyHostToDevice, s));
-  FGPU_TRY(launch_pq_residuals(dx, dim, drows.p, actual, d_assign, d_cent, res.p, s));
+  FGPU_TRY(launch_pq_residuals(dx, dim, drows.p, actual, d_assign, d_cent, ncent, res.p, s));
   FGPU_TRY(launch_pq_init(res.p, actual, dim, pq_m, dinit.p, d_codebook, s));
   for (int it = 0; it < iters; ++it) {
     FGPU_TRY(launch_pq_estep(res.p, actual, dim, pq_m, d_codebook, dassign.p, s));
@@ -1472,7 +1472,7 @@ fgpu_status fgpu_pq_train(const float* dx, int64_t n, int dim, int pq_m, const i
   FGPU_CHECK(dx && d_assign && d_cent && d_codebook && n >= 1 && pq_m >= 1 && dim % pq_m == 0 && iters >= 0,
              FGPU_ERR_ARG, "pq_train: bad argument");
   FGPU_CHECK(std::min<int64_t>(sample_size, n) >= kPQK, FGPU_ERR_ARG, "pq_train: need at least 256 sample rows");
-  return pq_train_sampled(dx, dim, pq_m, d_assign, d_cent, PqSample(n, pq_m, sample_size), iters, d_codebook,
+  return pq_train_sampled(dx, dim, pq_m, d_assign, d_cent, INT_MAX, PqSample(n, pq_m, sample_size), iters, d_codebook,
                           as_stream(stream));
 }
 
@@ -1540,6 +1540,9 @@ fgpu_status fgpu_build_ivfpq_sampled(const float* dx, int64_t n, int dim, int nl
     FGPU_TRY(fgpu_l2_topk(dx, n, cent.p, nlist, dim, 1, assign.p, dist.p, tws.p, tb, stream));
     FGPU_HIP(hipStreamSynchronize(s));
   }
+  FGPU_CHECK(pq_ok && pq_iters >= 0, FGPU_ERR_ARG, "build: pq_m must divide dim, pq_iters >= 0 and 256 sample rows or more");
+  FGPU_TRY(pq_train_sampled(dx, dim, pq_m, assign.p, cent.p, nlist,
+                            sample.valid() ? sample.get() : PqSample(n, pq_m, sample_size), pq_iters, cb.p, s));
   // inverted lists in cluster order, ids ascending inside a list
   // (build_global.cu:225-240); the codes are written in that order
   DevBuf<int32_t> offs, ids, pos;
@@ -1550,22 +1553,17 @@ fgpu_status fgpu_build_ivfpq_sampled(const float* dx, int64_t n, int dim, int nl
   FGPU_TRY(pos.alloc(n));
   FGPU_TRY(lws.alloc(lb));
   FGPU_TRY(launch_list_order(assign.p, n, nlist, offs.p, ids.p, pos.p, lws.p, lb, s));
-  // A row without a finite distance to any centroid (NaN, or an overflow) has no
-  // list: PQ training and encoding would read past the centroids for it.
-  int32_t listed = 0;
-  FGPU_HIP(hipMemcpyAsync(&listed, offs.p + nlist, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-  FGPU_HIP(hipStreamSynchronize(s));
-  FGPU_CHECK(listed == n, FGPU_ERR_ARG, "build: " + std::to_string(n - listed) + " rows have no finite distance to a centroid");
-  FGPU_CHECK(pq_ok && pq_iters >= 0, FGPU_ERR_ARG, "build: pq_m must divide dim, pq_iters >= 0 and 256 sample rows or more");
-  FGPU_TRY(pq_train_sampled(dx, dim, pq_m, assign.p, cent.p, sample.valid() ? sample.get() : PqSample(n, pq_m, sample_size),
-                            pq_iters, cb.p, s));
-  FGPU_TRY(launch_pq_encode(dx, n, dim, pq_m, assign.p, cent.p, cb.p, codes.p, s, 1, pos.p));
+  FGPU_TRY(launch_pq_encode(dx, n, dim, pq_m, assign.p, cent.p, cb.p, codes.p, s, 1, nlist, pos.p));
   FGPU_HIP(hipMemcpyAsync(h_offsets, offs.p, sizeof(int32_t) * ((size_t)nlist + 1), hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipMemcpyAsync(h_ids, ids.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipMemcpyAsync(h_codes, codes.p, (size_t)n * pq_m, hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipMemcpyAsync(h_centroids, cent.p, sizeof(float) * (size_t)nlist * dim, hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipMemcpyAsync(h_codebook, cb.p, sizeof(float) * (size_t)pq_m * kPQK * (dim / pq_m), hipMemcpyDeviceToHost, s));
   FGPU_HIP(hipStreamSynchronize(s));
+  // A row without a finite distance to any centroid (NaN, or an overflow) has no
+  // list; the kernels above pass over its assignment (INT_MAX).
+  FGPU_CHECK(h_offsets[nlist] == n, FGPU_ERR_ARG,
+             "build: " + std::to_string(n - h_offsets[nlist]) + " rows have no finite distance to a centroid");
   return FGPU_OK;
 }
 

@@ -437,17 +437,20 @@ fgpu_status launch_kmeans_finalize(const unsigned long long* sums, const int32_t
 fgpu_status launch_gather_rows(const float* x, int dim, const int32_t* rows, int nrows, float* out,
                                hipStream_t s);
 // fma_mode 1: the device form (fused chain); 0: the host form (separate roundings).
-// pos (may be null): row i's codes go to row pos[i] of codes.
+// ncent: the centroids (an assignment past them, a row without a centre, is read
+// as 0).  pos (may be null): row i's codes go to row pos[i] of codes, nowhere if it
+// is below 0.
 fgpu_status launch_pq_encode(const float* x, int64_t n, int dim, int m, const int32_t* assign,
                              const float* cent, const float* codebook, uint8_t* codes, hipStream_t s,
-                             int fma_mode = 1, const int32_t* pos = nullptr);
+                             int fma_mode = 1, int ncent = INT_MAX, const int32_t* pos = nullptr);
 // The inverted lists of an assignment: offsets[nlist + 1], ids in list order
-// (ascending inside a list) and each row's place in it.
+// (ascending inside a list) and each row's place in it (-1 for a row whose
+// assignment is out of range; offsets[nlist] is then below n).
 size_t list_order_ws_bytes(int64_t n, int nlist);
 fgpu_status launch_list_order(const int32_t* assign, int64_t n, int nlist, int32_t* offsets, int32_t* ids,
                               int32_t* pos, void* ws, size_t ws_bytes, hipStream_t s);
 fgpu_status launch_pq_residuals(const float* x, int dim, const int32_t* rows, int nrows,
-                                const int32_t* assign, const float* cent, float* res, hipStream_t s);
+                                const int32_t* assign, const float* cent, int ncent, float* res, hipStream_t s);
 fgpu_status launch_pq_init(const float* res, int nsample, int dim, int m, const int32_t* init_rows,
                            float* codebook, hipStream_t s);
 // assign_pq: pq_assign_bytes(nsample, m) bytes, 16-byte aligned.
