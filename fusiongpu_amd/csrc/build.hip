@@ -259,8 +259,9 @@ __device__ __forceinline__ float pq_dist(const float (&r)[S], const float* p) {
 // leading block is looked through once more at the end, instead of a compare
 // and two selects a codeword.  Each codeword read serves R vectors.  VALU bounds
 // both callers, then LDS: 500k x 32 codes of 4 dims encoded in 1231 -> 938 us, an
-// E step of 50k rows 114 -> 102 us.  cw: codeword k at cw + k * stride.
-constexpr int kPQBlock = 16, kPQRows = 2;
+// E step of 50k rows 114 -> 102 us.  R is 2, or 1 for calls that leave threads
+// idle (the launches' rules).  cw: codeword k at cw + k * stride.
+constexpr int kPQBlock = 16;
 template <int S, bool FMA, int R>
 __device__ __forceinline__ void pq_nearest(const float (&r)[R][S], const float* cw, int stride, int (&out)[R]) {
   float best[R];
@@ -309,10 +310,10 @@ __device__ __forceinline__ void pq_nearest(const float (&r)[R][S], const float* 
 // form, dist = fmaf(diff, diff, dist) as nvcc contracts encode_residuals_kernel
 // (kmeans_gpu.cuh:428-433); otherwise the host form of encode_residuals_to_pq
 // (pq_utils.h:160-166, built without FMA): the product and the sum each rounded.
-// A thread takes the same subspace of kPQRows rows; one workgroup a CU, as the
-// codebook fills its LDS, each staging it once.
+// A thread takes the same subspace of R rows; one workgroup a CU, as the codebook
+// fills its LDS, each staging it once.
 // pos (may be null): row i's codes go to row pos[i], nowhere if it is below 0.
-template <int S, bool FMA>
+template <int S, bool FMA, int R>
 __global__ __launch_bounds__(1024) void pq_encode_kernel(const float* __restrict__ x, int64_t n, int dim, int m,
                                                          const int32_t* __restrict__ assign,
                                                          const float* __restrict__ cent, uint32_t ncent,
@@ -325,13 +326,13 @@ __global__ __launch_bounds__(1024) void pq_encode_kernel(const float* __restrict
     cbs[t] = codebook[((size_t)sub * kPQK + kk) * S + j];
   }
   __syncthreads();
-  const int64_t total = (n + kPQRows - 1) / kPQRows * m;
+  const int64_t total = (n + R - 1) / R * m;
   for (int64_t pr = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; pr < total; pr += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i0 = pr / m * kPQRows;
+    const int64_t i0 = pr / m * R;
     const int sub = (int)(pr % m);
-    float r[kPQRows][S];
+    float r[R][S];
 #pragma unroll
-    for (int q = 0; q < kPQRows; ++q) {
+    for (int q = 0; q < R; ++q) {
       const int64_t i = min(i0 + q, n - 1);
       const float* xi = x + i * dim + sub * S;
       const uint32_t c = (uint32_t)assign[i];
@@ -339,10 +340,10 @@ __global__ __launch_bounds__(1024) void pq_encode_kernel(const float* __restrict
 #pragma unroll
       for (int j = 0; j < S; ++j) r[q][j] = xi[j] - ci[j];
     }
-    int bk[kPQRows];
-    pq_nearest<S, FMA, kPQRows>(r, cbs + sub * S, m * S, bk);
+    int bk[R];
+    pq_nearest<S, FMA, R>(r, cbs + sub * S, m * S, bk);
 #pragma unroll
-    for (int q = 0; q < kPQRows; ++q)
+    for (int q = 0; q < R; ++q)
       if (i0 + q < n) {
         const int64_t to = pos ? (int64_t)pos[i0 + q] : i0 + q;
         if (to >= 0) codes[to * m + sub] = (uint8_t)bk[q];
@@ -444,7 +445,7 @@ __global__ void pq_init_kernel(const float* __restrict__ res, int dim, int m, in
 
 // E-step of run_kmeans_pq_fast (pq_utils.h:39-52), host floating point: the
 // square and the running sum are rounded separately (no fused multiply-add).
-template <int S>
+template <int S, int R>
 __global__ __launch_bounds__(256) void pq_estep_kernel(const float* __restrict__ res, int ns, int dim, int m,
                                                        const float* __restrict__ codebook,
                                                        uint8_t* __restrict__ assign_pq, int stride) {
@@ -452,17 +453,17 @@ __global__ __launch_bounds__(256) void pq_estep_kernel(const float* __restrict__
   const int sub = blockIdx.y;
   for (int t = threadIdx.x; t < kPQK * S; t += blockDim.x) cbs[t] = codebook[(size_t)sub * kPQK * S + t];
   __syncthreads();
-  const int i0 = blockIdx.x * 256 * kPQRows + threadIdx.x;
+  const int i0 = blockIdx.x * 256 * R + threadIdx.x;
   if (i0 >= ns) return;
-  float xv[kPQRows][S];
+  float xv[R][S];
 #pragma unroll
-  for (int q = 0; q < kPQRows; ++q)
+  for (int q = 0; q < R; ++q)
 #pragma unroll
     for (int j = 0; j < S; ++j) xv[q][j] = res[(int64_t)min(i0 + 256 * q, ns - 1) * dim + sub * S + j];
-  int bc[kPQRows];
-  pq_nearest<S, false, kPQRows>(xv, cbs, S, bc);
+  int bc[R];
+  pq_nearest<S, false, R>(xv, cbs, S, bc);
 #pragma unroll
-  for (int q = 0; q < kPQRows; ++q)
+  for (int q = 0; q < R; ++q)
     if (i0 + 256 * q < ns) assign_pq[(size_t)sub * stride + i0 + 256 * q] = (uint8_t)bc[q];
 }
 
@@ -1048,21 +1049,25 @@ fgpu_status launch_pq_encode(const float* x, int64_t n, int dim, int m, const in
   const size_t lds = (size_t)kPQK * dim * sizeof(float);
   FGPU_CHECK(lds <= 160 * 1024, FGPU_ERR_UNSUPPORTED, "pq_encode: codebook exceeds LDS");
   if (n <= 0) return FGPU_OK;
-  const int64_t pairs = (n + kPQRows - 1) / kPQRows * m;
-  const unsigned grid = (unsigned)std::min<int64_t>((pairs + 1023) / 1024, 256);
-#define FGPU_ENC(SS, F)                                                                                       \
-  if (S == SS && (fma_mode != 0) == F) {                                                                      \
-    FGPU_HIP(hipFuncSetAttribute((const void*)pq_encode_kernel<SS, F>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                 (int)lds));                                                                  \
-    hipLaunchKernelGGL((pq_encode_kernel<SS, F>), dim3(grid), dim3(1024), lds, s, x, n, dim, m, assign, cent, (uint32_t)ncent, \
-                       codebook, pos, codes);                                                                         \
+  // Two rows a thread, unless one row each leaves none of the 256 x 1024 threads a
+  // second turn: then a thread's own work is the time.  Measured (us, two / one row
+  // a thread, 128 dims): 1000 rows, 32 codes 39 / 30, 16 codes 59 / 46; 16000 rows,
+  // 16 codes 61 / 50, 32 codes 44 / 61; 40000 rows, 16 codes 108 / 136.
+  const int rows = n * m <= 256 * 1024 ? 1 : 2;
+  const int64_t units = (n + rows - 1) / rows * m;
+  const unsigned grid = (unsigned)std::min<int64_t>((units + 1023) / 1024, 256);
+#define FGPU_ENC(SS, F, RR)                                                                                   \
+  if (S == SS && (fma_mode != 0) == F && rows == RR) {                                                        \
+    FGPU_HIP(hipFuncSetAttribute((const void*)pq_encode_kernel<SS, F, RR>,                                    \
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                      \
+    hipLaunchKernelGGL((pq_encode_kernel<SS, F, RR>), dim3(grid), dim3(1024), lds, s, x, n, dim, m, assign, cent, \
+                       (uint32_t)ncent, codebook, pos, codes);                                                                 \
     FGPU_HIP(hipGetLastError());                                                                              \
     return FGPU_OK;                                                                                           \
   }
-  FGPU_ENC(1, true) FGPU_ENC(2, true) FGPU_ENC(3, true) FGPU_ENC(4, true) FGPU_ENC(6, true) FGPU_ENC(8, true)
-  FGPU_ENC(16, true)
-  FGPU_ENC(1, false) FGPU_ENC(2, false) FGPU_ENC(3, false) FGPU_ENC(4, false) FGPU_ENC(6, false) FGPU_ENC(8, false)
-  FGPU_ENC(16, false)
+#define FGPU_ENC_S(SS) FGPU_ENC(SS, true, 1) FGPU_ENC(SS, true, 2) FGPU_ENC(SS, false, 1) FGPU_ENC(SS, false, 2)
+  FGPU_ENC_S(1) FGPU_ENC_S(2) FGPU_ENC_S(3) FGPU_ENC_S(4) FGPU_ENC_S(6) FGPU_ENC_S(8) FGPU_ENC_S(16)
+#undef FGPU_ENC_S
 #undef FGPU_ENC
   return set_error(FGPU_ERR_UNSUPPORTED, "pq_encode: unsupported sub-dimension");
 }
@@ -1084,18 +1089,25 @@ fgpu_status launch_pq_init(const float* res, int nsample, int dim, int m, const 
 static int pq_stride(int ns) { return (ns + 15) / 16 * 16; }
 size_t pq_assign_bytes(int ns, int m) { return (size_t)pq_stride(ns) * m; }
 
+// Workgroups of 256 threads up to which the E step takes one row a thread: three a
+// CU run together.  Measured (us an iteration with its M step, two rows / one):
+// 500 rows, 16 codes 37.5 / 25.6; 4000 rows, 48 codes 25.4 / 21.8 (768
+// workgroups); 16000 rows, 16 codes 56.5 / 59.6 (1008).
+constexpr int kEstepOneRow = 768;
 fgpu_status launch_pq_estep(const float* res, int ns, int dim, int m, const float* codebook, uint8_t* assign_pq,
                             hipStream_t s) {
   const int S = dim / m;
-  dim3 grid((unsigned)((ns + 256 * kPQRows - 1) / (256 * kPQRows)), (unsigned)m);
-#define FGPU_EST(SS)                                                                                     \
-  if (S == SS) {                                                                                         \
-    hipLaunchKernelGGL(pq_estep_kernel<SS>, grid, dim3(256), 0, s, res, ns, dim, m, codebook, assign_pq, \
-                       pq_stride(ns));                                                                   \
-    FGPU_HIP(hipGetLastError());                                                                         \
-    return FGPU_OK;                                                                                      \
+  const int rows = (int64_t)((ns + 255) / 256) * m <= kEstepOneRow ? 1 : 2;
+  const dim3 grid((unsigned)((ns + 256 * rows - 1) / (256 * rows)), (unsigned)m);
+#define FGPU_EST(SS, RR)                                                                                      \
+  if (S == SS && rows == RR) {                                                                                \
+    hipLaunchKernelGGL((pq_estep_kernel<SS, RR>), grid, dim3(256), 0, s, res, ns, dim, m, codebook, assign_pq, \
+                       pq_stride(ns));                                                                        \
+    FGPU_HIP(hipGetLastError());                                                                              \
+    return FGPU_OK;                                                                                           \
   }
-  FGPU_EST(1) FGPU_EST(2) FGPU_EST(3) FGPU_EST(4) FGPU_EST(6) FGPU_EST(8) FGPU_EST(16)
+  FGPU_EST(1, 1) FGPU_EST(2, 1) FGPU_EST(3, 1) FGPU_EST(4, 1) FGPU_EST(6, 1) FGPU_EST(8, 1) FGPU_EST(16, 1)
+  FGPU_EST(1, 2) FGPU_EST(2, 2) FGPU_EST(3, 2) FGPU_EST(4, 2) FGPU_EST(6, 2) FGPU_EST(8, 2) FGPU_EST(16, 2)
 #undef FGPU_EST
   return set_error(FGPU_ERR_UNSUPPORTED, "pq_estep: unsupported sub-dimension");
 }

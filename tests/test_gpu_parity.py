@@ -591,6 +591,26 @@ def test_pq_encode_ties_and_extremes(n, dim, m):
     assert np.array_equal(_host(got), oracle.pq_encode(x, a, cent, cb, fma_mode=1))
 
 
+@pytest.mark.parametrize("n,dim,m", [(8192, 128, 32), (8193, 128, 32), (2731, 96, 96), (2730, 96, 96), (16385, 96, 16)])
+def test_pq_rows_a_thread_edges(n, dim, m):
+    """Row counts on both sides of the lines between one and two rows a thread, in encoding (256 x 1024 codes) and
+    in the training's E step (768 workgroups)."""
+    _say(f"pq rows a thread n={n} dim={dim} m={m}")
+    rng = np.random.default_rng(n + m)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    a = rng.integers(0, 4, n).astype(np.int32)
+    cent = rng.standard_normal((4, dim)).astype(np.float32)
+    ns = 768 // m * 256
+    dx, da, dc = (torch.from_numpy(v).cuda() for v in (x, a, cent))
+    for rows in (min(n, ns), min(n, ns + 1)):
+        cb = fg.pq_train(dx[:rows], da[:rows], dc, m, sample_size=rows, iters=2)
+        want = oracle.pq_train(x[:rows], a[:rows], cent, m, sample_size=rows, iters=2)
+        assert np.array_equal(_bits(_host(cb)), _bits(want))
+    for mode in (0, 1):
+        got = fg.pq_encode(dx, da, dc, cb, fma_mode=mode)
+        assert np.array_equal(_host(got), oracle.pq_encode(x, a, cent, want, fma_mode=mode))
+
+
 @pytest.mark.parametrize("n,nlist,distinct", [(256, 1, 256), (2048, 7, 2048), (2049, 300, 40), (6145, 33, 6145)])
 def test_build_lists_at_chunk_edges(n, nlist, distinct):
     """The inverted lists at the edges of the 2048-row chunks they are sorted in: one list, a chunk of one row,
