@@ -438,7 +438,7 @@ fgpu_status launch_assign_d(const float* x, int64_t n, const float* c, int nc, c
 
 bool assign_takes(const float* x, int64_t n, const float* c, int nc, int dim, size_t ws_bytes) {
   if (((uintptr_t)x & 15) || ((uintptr_t)c & 15) || nc < kAssignMinCols || nc > kAssignMaxCols ||
-      n < kAssignMinRows)
+      n < (dim > 64 && nc <= kAssignFewCols ? kAssignMinRowsFewCols : kAssignMinRows))
     return false;
   if (dim != 32 && dim != 64 && dim != 96 && dim != 128) return false;
   const int64_t tiles = (nc + 31) / 32;

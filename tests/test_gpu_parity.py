@@ -163,7 +163,7 @@ def test_l2_topk_nearest_extremes(case):
     assert np.array_equal(_host(ids).view(np.uint32), oid) and np.array_equal(_bits(_host(d)), _bits(od))
 
 
-@pytest.mark.parametrize("dim,nc", [(128, 64), (96, 1024), (32, 100)])
+@pytest.mark.parametrize("dim,nc", [(64, 64), (128, 1024), (32, 100)])
 def test_l2_topk_nearest_overflowing_distances(dim, nc):
     """Finite rows whose squared distances overflow, to every column (the first one then, at distance inf) or to all but
     a few equally large ones, beside ordinary rows."""
@@ -199,6 +199,20 @@ def test_l2_topk_nearest_near_subnormal_distances(dim, e):
     ids, d = fg.l2_topk(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), 1)
     oid, od = oracle.coarse(x, c, 1, prune_ratio=np.inf)
     assert np.array_equal(_bits(_host(d)), _bits(od)) and np.array_equal(_host(ids).view(np.uint32), oid)
+
+
+@pytest.mark.parametrize("n,dim,nc", [(32767, 128, 129), (32768, 128, 129), (40959, 128, 128), (40960, 128, 128),
+                                      (40960, 96, 32), (32768, 64, 32), (32768, 64, 31)])
+def test_l2_topk_nearest_route_edges(n, dim, nc):
+    """Row and column counts on both sides of the lines between the register-resident pass and the estimate + select
+    pair: the oracle's answer either way."""
+    _say(f"l2_topk nearest route edges n={n} dim={dim} nc={nc}")
+    rng = np.random.default_rng(n + nc)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    c = rng.standard_normal((nc, dim)).astype(np.float32)
+    ids, d = fg.l2_topk(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), 1)
+    oid, od = oracle.coarse(x, c, 1, prune_ratio=np.inf)
+    assert np.array_equal(_host(ids).view(np.uint32), oid) and np.array_equal(_bits(_host(d)), _bits(od))
 
 
 # --------------------------------------------------------------------------- coarse quantizer (A2, A3)
