@@ -158,9 +158,9 @@ __device__ __forceinline__ void assign_stage(const uint4* __restrict__ cur, uint
 // 2 (D / 16 + 1) MFMAs of 32 cycles (576 at D = 128) against 96 VALU
 // instructions of 4 for the two smallest keys (insert the tile number, median,
 // minimum), which the other wave of the SIMD overlaps.  Two row sets halve the
-// LDS reads an MFMA needs.  Measured, 1M rows x 4096 columns x 128 dims: 1.24 ms
-// = 846 TFLOP/s (950 with the extra block; a large bf16 product reaches 1177 on
-// the same card), the rescore 0.41 ms; one Lloyd step 10.6 -> 2.5 ms against the
+// LDS reads an MFMA needs.  Measured, 1M rows x 4096 columns x 128 dims: 1.13 ms
+// = 930 TFLOP/s (1050 with the extra block; a large bf16 product reaches 1177 on
+// the same card), the rescore 0.20 ms; one Lloyd step 10.4 -> 1.46 ms against the
 // estimate + select pair (three bf16 products, 8 GB of estimates).
 template <int D>
 __global__ __launch_bounds__(kAWaves * kWave, 2) void assign_kernel(const float* __restrict__ x, int64_t n, int nc,
@@ -338,12 +338,66 @@ __device__ __forceinline__ float wave_pairs_l2(const float* __restrict__ x, cons
   return acc;
 }
 
+// Every column's exact distance for the wave's 64 rows, a lane a row: each lane's
+// smallest (distance, column) key, kNoKey if every distance is NaN.  A column's
+// values are the same for the whole wave and come through scalar loads; the row is
+// read once every kDenseCols columns.  VALU bounds it: 84 G pairs of 128 dims a
+// second (200,000 rows x 1024 columns 2.43 ms), pair by pair about 20 G.
+constexpr uint64_t kNoKey = ((uint64_t)0x7F800000u << 32) | (uint32_t)kPadId;  // above every key that is not NaN
+constexpr int kDenseCols = 16;
+template <int D>
+__device__ __forceinline__ uint64_t wave_all_columns(const float* __restrict__ xr, const float* __restrict__ c, int nc) {
+  uint64_t best = kNoKey;
+#pragma unroll 1
+  for (int c0 = 0; c0 < nc; c0 += kDenseCols) {
+    float acc[kDenseCols];
+#pragma unroll
+    for (int j = 0; j < kDenseCols; ++j) acc[j] = 0.0f;
+#pragma unroll 1
+    for (int l = 0; l < D / 32; ++l) {
+      float4 v[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) v[t] = reinterpret_cast<const float4*>(xr)[8 * l + t];
+#pragma unroll
+      for (int j = 0; j < kDenseCols; ++j) {
+        const float4* cr = reinterpret_cast<const float4*>(c + (size_t)min(c0 + j, nc - 1) * D + 32 * l);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const float4 w = cr[t];
+          float df = v[t].x - w.x;
+          acc[j] = __builtin_fmaf(df, df, acc[j]);
+          df = v[t].y - w.y;
+          acc[j] = __builtin_fmaf(df, df, acc[j]);
+          df = v[t].z - w.z;
+          acc[j] = __builtin_fmaf(df, df, acc[j]);
+          df = v[t].w - w.w;
+          acc[j] = __builtin_fmaf(df, df, acc[j]);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kDenseCols; ++j) {
+      const uint64_t key = key_of(acc[j], c0 + j);
+      best = c0 + j < nc && key < best ? key : best;
+    }
+  }
+  return best;
+}
+
 // The candidates' exact distances: a wave takes 64 rows, packs their candidate
 // columns 64 at a time and keeps each row's smallest (distance, column) key.
 // A row all of whose distances overflow has its first column, at distance inf; one
 // that is not finite itself (no candidates) has none (kPadKey).
+// Where the wave's entries name more than a kDenseShare-th of its pairs (data whose
+// common offset is far larger than its differences, equal columns) every pair is
+// computed instead: 200,000 rows x 1024 columns 20 -> 2.4 ms, 50,000 x 4096 (one
+// wave a SIMD) 26 -> 9.4, both 11.2 with the estimate + select pair.  (Both forms
+// cost the same near a quarter of the pairs with many waves, later with one a SIMD.)
+// The lambdas are always_inline: left to the compiler, what they capture lay in
+// scratch memory and each batch waited for it, 384 us against 201 (1M rows x 4096
+// columns, 128 dims).
 constexpr int kRWaves = 4;
-constexpr uint64_t kNoKey = ((uint64_t)0x7F800000u << 32) | (uint32_t)kPadId;  // above every key that is not NaN
+constexpr int kDenseShare = 3;
 template <int D>
 __global__ __launch_bounds__(kRWaves * kWave, 4) void assign_rescore_kernel(
     const float* __restrict__ x, int64_t n, const float* __restrict__ c, int nc, const uint16_t* __restrict__ cand,
@@ -358,10 +412,10 @@ __global__ __launch_bounds__(kRWaves * kWave, 4) void assign_rescore_kernel(
   unsigned long long* best = best_s[wave];
   uint32_t* q = q_s[wave];  // row << 16 | column
   const int64_t row = row0 + lane;
-  const int ncand = row < n ? (int)cnt[row] : 0;
+  int ncand = row < n ? (int)cnt[row] : 0;
   best[lane] = kNoKey;
   int nq = 0;
-  auto score = [&](int m) {
+  auto score = [&](int m) __attribute__((always_inline)) {
     wave_lds_order();
     const uint32_t e = q[lane < m ? lane : 0];
     const int rl = (int)(e >> 16), col = (int)(e & 0xFFFFu);
@@ -370,7 +424,7 @@ __global__ __launch_bounds__(kRWaves * kWave, 4) void assign_rescore_kernel(
     wave_lds_order();
   };
   // Append a column for each lane with `f`; a full wave of them is scored.
-  auto push = [&](bool f, uint32_t e) {
+  auto push = [&](bool f, uint32_t e) __attribute__((always_inline)) {
     const uint64_t bm = __ballot(f);
     if (f) q[nq + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u))] = e;
     nq += __popcll(bm);
@@ -382,6 +436,16 @@ __global__ __launch_bounds__(kRWaves * kWave, 4) void assign_rescore_kernel(
       nq -= kWave;
     }
   };
+  // Counted only where a third of the rows have candidates in half the classes.
+  if (__builtin_expect(__popcll(__ballot(ncand >= kASlots / 2)) * kDenseShare >= kWave, 0)) {
+    int cols = 0;
+    for (int s = 0; s < ncand; ++s) cols += cand[row * kASlots + s] & kAClass ? (nc + 31) / 32 : 1;
+    if (wave_sum_i(cols) * kDenseShare > nc * kWave) {
+      const uint64_t b = wave_all_columns<D>(x + min(row, n - 1) * D, c, nc);
+      if (ncand > 0) best[lane] = b;
+      ncand = 0;
+    }
+  }
   for (int s = 0; __ballot(s < ncand); ++s) {
     const uint32_t e = s < ncand ? cand[row * kASlots + s] : 0u;
     const bool cls = s < ncand && (e & kAClass);
@@ -438,7 +502,7 @@ fgpu_status launch_assign_d(const float* x, int64_t n, const float* c, int nc, c
 
 bool assign_takes(const float* x, int64_t n, const float* c, int nc, int dim, size_t ws_bytes) {
   if (((uintptr_t)x & 15) || ((uintptr_t)c & 15) || nc < kAssignMinCols || nc > kAssignMaxCols ||
-      n < (dim > 64 && nc <= kAssignFewCols ? kAssignMinRowsFewCols : kAssignMinRows))
+      n < kAssignMinRows)
     return false;
   if (dim != 32 && dim != 64 && dim != 96 && dim != 128) return false;
   const int64_t tiles = (nc + 31) / 32;

@@ -53,18 +53,16 @@ fgpu_status launch_select_exact(const void* est, int64_t ld, int64_t nrows, int 
 // The nearest column of every row (p = 1) without an estimate matrix
 // (assign.hip): ids and exact distances; ws holds its column tiles and each
 // row's candidates.  assign_takes: whether it applies (dim 32, 64, 96 or 128,
-// 16-byte aligned arrays, at least kAssignMinRows rows, or kAssignMinRowsFewCols
-// where columns are few and wide, kAssignMinCols to kAssignMaxCols columns, room
-// for 512 rows) rather than the estimate + select pair.  A workgroup walks every
-// column, so below about 64 workgroups (512 rows each) the pair, which also splits
-// the columns, is faster, and with few columns its own start-up shows.  Measured
-// (us, pair / this, dim 128): 8192 rows 29 / 51 (256 columns) and 92 / 139 (4096);
-// 32768 rows 48 / 57 (32 columns), 55 / 59 (128), 65 / 62 (256); 40960 rows 57 / 57,
-// 65 / 60, 77 / 64; 65,536 rows 120 / 61 (256) and 624 / 158 (4096); 262,144 rows
-// 423 / 118 and 2486 / 360; 32768 rows of 64 dims 33 / 34 (32), 40 / 36 (128); 65,536
-// rows of 16 columns 87 / 85.
-constexpr int kAssignMinCols = 32, kAssignFewCols = 128, kAssignMaxCols = 4096;
-constexpr int64_t kAssignMinRows = 32768, kAssignMinRowsFewCols = 40960;
+// 16-byte aligned arrays, at least kAssignMinRows rows, kAssignMinCols to
+// kAssignMaxCols columns, room for 512 rows) rather than the estimate + select
+// pair.  A workgroup walks every column, so below about 64 workgroups (512 rows
+// each) the pair, which also splits the columns, is faster, and with fewer than a
+// tile of columns the rest of it is work for padding.  Measured (us, pair / this,
+// dim 128): 16384 rows 41 / 49 (256 columns) and 165 / 158 (4096); 24576 rows 39 / 45
+// (32), 54 / 52 (256); 32768 rows 47 / 74 (16), 48 / 46 (32), 65 / 53 (256) and 314 /
+// 158 (4096); 262,144 rows 422 / 109 and 2476 / 364.
+constexpr int kAssignMinCols = 32, kAssignMaxCols = 4096;
+constexpr int64_t kAssignMinRows = 32768;
 bool assign_takes(const float* x, int64_t n, const float* c, int nc, int dim, size_t ws_bytes);
 fgpu_status launch_assign(const float* x, int64_t n, const float* c, int nc, int dim, const float* cn_max, void* ws,
                           size_t ws_bytes, int32_t* ids, float* d, hipStream_t s);

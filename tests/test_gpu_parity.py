@@ -201,6 +201,36 @@ def test_l2_topk_nearest_near_subnormal_distances(dim, e):
     assert np.array_equal(_bits(_host(d)), _bits(od)) and np.array_equal(_host(ids).view(np.uint32), oid)
 
 
+@pytest.mark.parametrize("dim,nc", [(128, 33), (96, 100), (64, 1025), (32, 4096)])
+def test_l2_topk_nearest_dense_candidates(dim, nc):
+    """Waves of 64 rows with every column a candidate (a common offset far above the differences; equal columns), with
+    a few such rows and with none, column counts off the dense form's 16: the oracle's answer, ties to the lowest
+    column.  Some dense rows are not finite, some have only overflowing distances."""
+    _say(f"l2_topk nearest dense dim={dim} nc={nc}")
+    rng = np.random.default_rng(dim + nc)
+    off = np.float32(2000.0)
+    x = rng.standard_normal((32768, dim)).astype(np.float32)
+    c = (rng.standard_normal((nc, dim)) + off).astype(np.float32)
+    c[nc // 2:nc // 2 + 5] = c[3]
+    x[: 20000] += off
+    x[20000:20500:7] += off
+    x[64:128] = c[3]
+    x[130:140] *= np.float32(1e17)
+    n = 4096 if nc > 2000 else 32768  # rows the oracle checks
+    ids, d = fg.l2_topk(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), 1)
+    oid, od = oracle.coarse(x[-n // 2:], c, 1, prune_ratio=np.inf)
+    fid, fd = oracle.coarse(x[:n // 2], c, 1, prune_ratio=np.inf)
+    ids, d = _host(ids).view(np.uint32), _host(d)
+    assert np.array_equal(_bits(d[:n // 2]), _bits(fd)) and np.array_equal(ids[:n // 2], fid)
+    assert np.array_equal(_bits(d[-n // 2:]), _bits(od)) and np.array_equal(ids[-n // 2:], oid)
+    x[140], x[141, 0] = np.nan, np.inf
+    rid, rd = fg.l2_topk(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), 1)
+    rid, rd = _host(rid).view(np.uint32), _host(rd)
+    assert np.all(rid[140:142] == 0x7FFFFFFF)
+    rid[140:142], rd[140:142] = ids[140:142], d[140:142]
+    assert np.array_equal(rid, ids) and np.array_equal(_bits(rd), _bits(d))
+
+
 @pytest.mark.parametrize("n,dim,nc", [(32767, 128, 129), (32768, 128, 129), (40959, 128, 128), (40960, 128, 128),
                                       (40960, 96, 32), (32768, 64, 32), (32768, 64, 31)])
 def test_l2_topk_nearest_route_edges(n, dim, nc):
