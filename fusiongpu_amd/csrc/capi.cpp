@@ -270,15 +270,26 @@ struct ScreenWs {
   }
 };
 
+// Whether phase 1 of fgpu_two_phase_search takes the screen or stays in the
+// two-phase kernel: below 1024 queries the screen's fixed launches cost more than
+// they save there.  Codes of 3 or 6 dims (96 in 32 or 16) read more for each
+// decoded vector, so there the screen also needs long lists: about 2700 queries at
+// 1000 vectors a list, more on shorter ones, none below 450.  Measured (us, kernel /
+// screen, a whole batch, 20 probes, 12 phase-1 lists): 1000 vectors a list, 16 codes,
+// 2048 queries 235 / 226, 3072 324 / 273, 5000 477 / 379 (4 phase-1 lists 179 / 195,
+// 247 / 230, 370 / 294); 586 a list, 3072 queries 194 / 253, 5000 278 / 340, 32 codes
+// 202 / 223 and 292 / 300; 333 a list, 16 codes, 5000 200 / 265.
+constexpr int kTpScreenMinQueries = 1024, kTpScreen3MinQueries = 2048, kTpScreen3MinList = 450;
+constexpr int64_t kTpScreen3Work = 1500000;
+bool tp_screen_pays(const fgpu_index* ix, int nq) {
+  if (ix->dim / ix->m % 3 != 0) return nq >= kTpScreenMinQueries;
+  return nq >= kTpScreen3MinQueries && nq * (ix->total / ix->nlist - kTpScreen3MinList) >= kTpScreen3Work;
+}
+
 // Phase 1 of fgpu_two_phase_search through the screen: the buffers of one
 // chunk of nvq virtual queries (one per (query, phase-1 probe); virtual query
 // v reads query row v / p1 of the chunk): their probes and (zero) probe distances, their top-limit_k results, the
 // per-list counts and compact bucket offsets, and the screen's workspace.
-// Batches below this many queries keep phase 1 in the two-phase kernel (the
-// screen's fixed launches cost more than they save there).
-// Codes of 3 or 6 dims: 2048 (96 dims, us, kernel / screen: 16 codes, 1024
-// queries 127 / 160, 2048 201 / 203, 5000 392 / 355; 64 probes 262 / 271, 481 / 375).
-constexpr int kTpScreenMinQueries = 1024, kTpScreen3MinQueries = 2048;
 constexpr int kTpVqMax = 131072;  // virtual queries a chunk (fuller 32-row MFMA groups per list)
 struct TpScreenWs {
   uint32_t* vprobe = nullptr;
@@ -949,8 +960,7 @@ fgpu_status two_phase(const fgpu_index* ix, const float* dq, int nq, const uint3
   // select.  The virtual queries' buffers take the end of the workspace; the
   // pools and cutoff rows the rest.
   const bool tp_screen = ix->opt_two_phase_screen == 2 ||
-                         (ix->opt_two_phase_screen == 0 &&
-                          nq >= (ix->dim / ix->m % 3 == 0 ? kTpScreen3MinQueries : kTpScreenMinQueries));
+                         (ix->opt_two_phase_screen == 0 && tp_screen_pays(ix, nq));
   if (tp_screen && ix->screen_ok && ix->opt_screen && limit_k <= 64 && p1 >= 1 && screen_supported(ix->dim, ix->m) &&
       ix->nlist <= kScreenMaxLists && ((uintptr_t)dq & 15) == 0) {
     // With FGPU_OPT_STAGE_EVENTS, the stage events of fgpu_search_stage_times

@@ -231,8 +231,9 @@ int fgpu_index_screen_ready(const fgpu_index* idx);
  *                       default;
  *   FGPU_OPT_TWO_PHASE_SCREEN phase 1 of fgpu_two_phase_search (limit_k <=
  *                       64) through the MFMA screen: 0 automatic (batches of
- *                       1024 queries or more), 1 never, 2 always; same
- *                       results;
+ *                       1024 queries or more; for 96 dims in 16 or 32 codes,
+ *                       of 2048 or more on lists long enough to pay), 1 never,
+ *                       2 always; same results;
  *   FGPU_OPT_SCREEN_CLOCKS 1: the screen kernels add their waves' shader
  *                       clocks (before the first item, item set-up, tile
  *                       loops, after the tiles; round 1 then round 2) to the
