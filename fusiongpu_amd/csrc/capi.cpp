@@ -212,16 +212,27 @@ constexpr int kSmallBatch = 64;
 //     blob (512 queries: 58 / 98 and 211 / 181);
 //   * up to 2048 for k > 32: k 64, 155 / 239 (2048 queries, C2's clusters), k 50
 //     in 16 codes of 96 dims, wide clusters: 559 / 1201;
-//   * codes of 3 or 6 dims (96 in 32 or 16): k <= 32 from 3072 queries on (48
-//     probes, 16 codes, 2000 queries 128 / 126, 4000 223 / 145; 32 codes 129 / 147
-//     and 224 / 170); past 64 probes, where one workgroup scans each query, from
-//     768 (32 codes, 100 probes, 512 queries 103 / 130, 1000 168 / 133).
-// Indexes below kScreenAnyBatch vectors keep the screen at every batch size: its
-// counters (fgpu_search_screen_stats) describe such searches.
-constexpr int kFlowRound = 256, kFlowWideK = 2048, kScreen3Flow = 3072, kScreen3Plain = 768;
+//   * codes of 3 or 6 dims (96 in 32 or 16): k <= 32 from 3072 queries on, more on
+//     lists of fewer than 500 vectors, where the screen's tiles are emptier (500,000
+//     in 1000 lists, 48 probes, 16 codes, 4096 queries 229 / 149; 1M in 1000, 32
+//     codes, 3072 179 / 130; 200,000 in 447, 3072 92 / 110, 6000 153 / 138; 70,000 in
+//     264, 3072 69 / 92, 6000 113 / 118); tight clusters in 16 codes favour the flow
+//     kernel longer (200,000 vectors, sigma 0.06, 6000 queries 141 / 208).  Past 64
+//     probes, where one workgroup scans each query, from 768 (32 codes, 100 probes,
+//     512 queries 103 / 130, 1000 168 / 133).
+// Indexes below kScreenAnyBatch vectors keep the screen for batches of more than
+// kSmallBatch queries (3072 for codes of 3 or 6 dims, whatever the lists), as programs and tests read its counters there
+// (fgpu_search_screen_stats); the flow kernel would often be faster (us, flow /
+// screen, 128 queries: 20,000 vectors, 128 dims in 32 codes, 32 probes 54 / 84;
+// 60,000, 34 / 71; in 64 codes 91 / 91 and 95 / 79).
+constexpr int kFlowRound = 256, kFlowWideK = 2048, kScreen3Flow = 3072, kScreen3List = 500, kScreen3Plain = 768;
 constexpr int64_t kScreenAnyBatch = 65536;
 bool screen_pays(const fgpu_index* ix, int nq, int k, bool flow) {
-  if (ix->dim / ix->m % 3 == 0) return flow ? k <= 32 && nq >= kScreen3Flow : nq >= kScreen3Plain;
+  if (ix->dim / ix->m % 3 == 0) {
+    const int64_t len = ix->total < kScreenAnyBatch ? kScreen3List
+                                                    : std::min<int64_t>(ix->total / ix->nlist, kScreen3List);
+    return flow ? k <= 32 && nq * len >= (int64_t)kScreen3Flow * kScreen3List : nq >= kScreen3Plain;
+  }
   return !flow || ix->total < kScreenAnyBatch || nq > (k > 32 ? kFlowWideK : kFlowRound);
 }
 
@@ -740,7 +751,8 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   auto mark = [&](int i) { return ev ? hipEventRecord(ev[i], s) : hipSuccess; };
   FGPU_HIP(mark(0));
   ScreenWs sw;
-  const bool flow = flow_grid(ix->dim, ix->m, nq, nprobe) > 0;
+  const int grid = flow_grid(ix->dim, ix->m, nq, nprobe);
+  const bool flow = grid > 0;
   // A small batch: coarse, then the LUT kernel with split probes
   // (launch_adc_hand) in the screen's buffers, beside the coarse step's tile.
   const size_t sbytes = nq <= kSmallBatch ? ScreenWs::bytes(nq, ix->nlist, nprobe) : 0;
@@ -810,7 +822,6 @@ fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprob
   }
   // The scan claims queries from a counter that starts at its grid size; the
   // coarse step's select stores that value on the way.
-  const int grid = flow_grid(ix->dim, ix->m, nq, nprobe);
   SelectSide side;
   side.ctr = qctr;
   side.ctr_val = grid;

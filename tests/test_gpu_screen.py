@@ -472,3 +472,17 @@ def test_screen_counters_follow_the_route(dim, m, nq, nprobe, k, screened):
     st = idx.search_screen_stats(nq, nprobe, ws)
     assert st["queries_to_lut_kernel"] == nq and not any(st[w] for w in work)
     idx.close()
+
+
+@pytest.mark.parametrize("m,nq,screened", [(16, 3071, False), (16, 3072, False), (16, 4000, True), (32, 2990, False),
+                                           (32, 4000, True)])
+def test_search_route_of_3_and_6_dims_weighs_the_lists(m, nq, screened):
+    """96 dims in 32 or 16 codes, 66,000 vectors in 170 lists (388 a list): 1,536,000 / 388 = 3959 queries take the
+    screen, fewer the flow kernel; the same results."""
+    _say(f"route 3/6 dims m={m} nq={nq}")
+    offs, ids, codes, cent, cb = _gmm_index(96, m, 170, 66000, seed=m)
+    idx = fg.Index.from_arrays(96, m, offs, ids, codes, cent, cb)
+    q = fg.gen_gmm(nq, 96, 32, seed=m, set=1, sig_lo=0.08)
+    st = _check(idx, q, cent, cb, offs, ids, codes, 6, 10)
+    assert (st["pairs_round1"] > 0) == screened
+    idx.close()
