@@ -968,7 +968,7 @@ fgpu_status launch_kmeans_accumulate(const float* x, int64_t n, const int32_t* a
   Carve cv(ows, ows_bytes);
   int32_t* cursor = cv.take<int32_t>((size_t)k + 1);
   int32_t* cnt = cv.take<int32_t>((size_t)k);  // this chunk's counts
-  const int64_t rows = std::min<int64_t>(n, fit);
+  const int64_t rows = std::min<int64_t>({n, fit, (int64_t)1 << 30});  // a chunk's row numbers are 32-bit
   int32_t* order = cv.take<int32_t>((size_t)rows);
   FGPU_CHECK(cv.ok(), FGPU_ERR_WORKSPACE, "kmeans_update: workspace too small");
   const size_t lds = (size_t)k * sizeof(int32_t);
