@@ -222,9 +222,9 @@ constexpr int kSmallBatch = 64;
 //     512 queries 103 / 130, 1000 168 / 133).
 // Indexes below kScreenAnyBatch vectors keep the screen for batches of more than
 // kSmallBatch queries (3072 for codes of 3 or 6 dims, whatever the lists), as programs and tests read its counters there
-// (fgpu_search_screen_stats); the flow kernel would often be faster (us, flow /
-// screen, 128 queries: 20,000 vectors, 128 dims in 32 codes, 32 probes 54 / 84;
-// 60,000, 34 / 71; in 64 codes 91 / 91 and 95 / 79).
+// (fgpu_search_screen_stats); the flow kernel would be faster (us, flow / screen,
+// 128 queries, 128 dims in 32 codes, 32 probes: 5000 vectors 55 / 86, 20,000 54 /
+// 84, 60,000 34 / 71).
 constexpr int kFlowRound = 256, kFlowWideK = 2048, kScreen3Flow = 3072, kScreen3List = 500, kScreen3Plain = 768;
 constexpr int64_t kScreenAnyBatch = 65536;
 bool screen_pays(const fgpu_index* ix, int nq, int k, bool flow) {
@@ -722,12 +722,17 @@ extern "C" {
 
 size_t fgpu_search_workspace_bytes(int nq, int nlist, int nprobe) {
   // The coarse step's estimate tile and the screen's buffers are never live
-  // at once, so they share one region (no screen beyond kScreenMaxLists lists).
-  const size_t screen = nlist <= kScreenMaxLists ? ScreenWs::bytes(nq, nlist, nprobe) : 0;
-  const size_t coarse = fgpu_coarse_workspace_bytes(nq, nlist);
-  // (A small batch's select sets up the scan's words while it reads the tile.)
+  // at once, so they share one region (no screen beyond kScreenMaxLists lists),
+  // but for a small batch, whose select sets up the scan's words while it reads
+  // the tile.  A larger batch's workspace also holds the smaller ones.
+  auto scan = [&](int q, bool beside) {
+    const size_t screen = nlist <= kScreenMaxLists ? ScreenWs::bytes(q, nlist, nprobe) : 0;
+    const size_t coarse = fgpu_coarse_workspace_bytes(q, nlist);
+    return beside ? coarse + screen : std::max(coarse, screen);
+  };
   return carve_bytes<uint32_t>((size_t)nq * nprobe) + carve_bytes<float>((size_t)nq * nprobe) +
-         carve_bytes<int>(kSearchWords) + (nq <= kSmallBatch ? coarse + screen : std::max(coarse, screen));
+         carve_bytes<int>(kSearchWords) +
+         (nq <= kSmallBatch ? scan(nq, true) : std::max(scan(nq, false), scan(kSmallBatch, true)));
 }
 
 fgpu_status fgpu_search(const fgpu_index* ix, const float* dq, int nq, int nprobe, int k, float prune_ratio,

@@ -36,6 +36,14 @@ def test_abi_version():
     assert fg.lib.fgpu_abi_version() == 1
 
 
+@pytest.mark.parametrize("nlist,nprobe", [(16, 1), (256, 16), (1024, 32), (4096, 64), (8192, 256), (20000, 8)])
+def test_search_workspace_holds_every_smaller_batch(nlist, nprobe):
+    """A workspace sized for the largest batch of a program serves its smaller batches: the size never falls as the
+    batch grows, also where small batches need the coarse tile beside the scan's buffers."""
+    sizes = [fg.lib.fgpu_search_workspace_bytes(nq, nlist, nprobe) for nq in range(1, 400)]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+
+
 @pytest.mark.parametrize("n,k", [(1, 1), (300, 256), (65536, 50000), (65537, 50000), (70001, 256),
                                  (1_000_000, 50000), (3_000_001, 50000)])
 def test_pq_sample_prefix_equals_full_shuffle(n, k):
