@@ -422,9 +422,9 @@ def main():
                      "mfma_tile_frac": round(scr_exec_flop / (scr_ms * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4),
                      "bytes_read_per_launch": scr_bytes,
                      "hbm_gbs": round(scr_bytes / (scr_ms * 1e-3) / 1e9, 1),
-                     "note": "the step's longest kernel: bf16 MFMA distance bounds of (query, vector) pairs; "
+                     "note": "the step's longest kernel: fp16 MFMA distance bounds of (query, vector) pairs; "
                              "achieved = 2 (dim + 16) flops per pair screened (the bound GEMM, K = dim plus a "
-                             "16-wide block of constants) / its event-timed duration, against the dense bf16 "
+                             "16-wide block of constants) / its event-timed duration, against the dense fp16 / bf16 "
                              "peak; mfma_tile_frac counts the 32 x 32 tiles it runs (a list's queries padded to "
                              "32 rows); bytes_read = codes + 16-byte block of each vector row a tile reads; "
                              "traffic = copy-calibrated FETCH_SIZE + WRITE_SIZE per launch "

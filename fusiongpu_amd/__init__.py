@@ -662,7 +662,8 @@ class Index:
         runs the LUT kernels), OPT_SCREEN_CLOCKS (1 = the screen records shader clocks),
         OPT_TWO_PHASE_SPLIT (phase-1 workgroups a query: 0 automatic, 1 never, s >= 2), OPT_STAGE_EVENTS
         (1 = search records HIP events between its stages, read by search_stage_times), OPT_TWO_PHASE_SCREEN
-        (two-phase phase 1 through the MFMA screen: 0 automatic for batches >= 1024, 1 never, 2 always).
+        (two-phase phase 1 through the MFMA screen: 0 automatic for batches >= 1024, fewer cases for codes of 3 and
+        6 dims, 1 never, 2 always).
         Results never depend on them; they change only this index's later calls."""
         _check(lib.fgpu_index_set_option(self._h, int(option), int(value)))
 
@@ -672,8 +673,8 @@ class Index:
         return bool(lib.fgpu_index_screen_ready(self._h))
 
     def search_screen_stats(self, nq: int, nprobe: int, workspace, stream=None) -> dict:
-        """Counters of the last search() on `workspace` that took the MFMA screen (fgpu_search_screen_stats;
-        waits for the stream)."""
+        """Counters of the last search() on `workspace` (fgpu_search_screen_stats; waits for the stream): a search
+        that the LUT kernels answered alone has nothing screened and every query in queries_to_lut_kernel."""
         st = (_c.c_longlong * 20)()
         with _on(stream):
             _check(lib.fgpu_search_screen_stats(self._h, nq, nprobe, _dev_ptr(workspace), _ws_check(workspace),

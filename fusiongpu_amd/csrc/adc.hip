@@ -278,8 +278,8 @@ __global__ __launch_bounds__(kNT) void adc_plain_kernel(AdcArgs a) {
 // the other parts through that key in global memory (a 64-bit atomic min; a
 // stale value only skips less).  The last part to arrive merges the parts'
 // sorted keys.  Measured on C2 shapes (8 handed queries of 10,000, 32
-// probes): 106 us with one workgroup a query and no bound, 32 us now; 206 of
-// 2000 queries at 128 probes and 64 subspaces: about 1.4 ms, 64 us now.
+// probes): 106 us with one workgroup a query and no bound, 22 us now; 204 of
+// 2000 queries at 128 probes and 64 subspaces: about 1.4 ms, 88 us now.
 constexpr int kHandProbes = 256;  // probes a query can have (the coarse step's limit)
 
 template <int D, int M>

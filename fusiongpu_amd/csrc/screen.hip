@@ -1043,7 +1043,7 @@ __global__ __launch_bounds__(kRW * kWave) void rescore_kernel(ScreenArgs a) {
     // More than 64 candidates: the 64 strongest go first (each lane's largest
     // m); the k-th distance they give drops most of the others before they are
     // scored.  10k queries, C2 shapes, 30 candidates on average and up to 1400:
-    // 58 -> 36 us; 2000 queries of 226 on average, k 64: 60 -> 41 us.
+    // 58 -> 39 us; 2000 queries of 224 on average, k 64: 60 -> 39 us.
     // Single-probe queries seldom have more than two batches: as they come.
     uint2 e = lane < ncand ? cq[lane] : make_uint2(0u, 0u);
     int own = 0;  // the batch e came from

@@ -184,15 +184,29 @@ fgpu_status fgpu_adc_search_stats(const fgpu_index* idx, const float* d_queries,
                                   void* stream);
 
 /* coarse + ADC in one call: the same results as fgpu_coarse_search followed
- * by fgpu_adc_search.  For k <= 64 on the geometries (dim, pq_m) = (128, 16),
- * (128, 32), (128, 64), (96, 48) the scan part runs as an MFMA screen with an
- * exact rescore (no per-(query, list) LUT): every query's first list gives an
- * upper bound T on its k-th distance, every probed vector whose rigorous lower
- * bound does not exceed T is rescored with the reference's direct ADC form
- * (gpu_global.cu:259-319, bit-identical to the LUT sum), and the few queries
- * it cannot settle (a first list shorter than k, more than 512 candidates)
- * are scanned by the LUT kernel.  That needs fgpu_search_workspace_bytes; a
- * smaller workspace that still holds the coarse step runs the LUT kernels. */
+ * by fgpu_adc_search.  Which kernels scan depends on the sizes (the rules and
+ * their times stand in capi.cpp); the results do not.  For k <= 64 on the
+ * geometries (dim, pq_m) = (128, 16), (128, 32), (128, 64), (96, 16), (96, 32),
+ * (96, 48):
+ *   up to 64 queries     a LUT kernel with every query's probes split over the
+ *                        GPU ((96, 16) and (96, 32) up to 64 probes: the flow
+ *                        kernel, one workgroup a query);
+ *   up to 64 probes,     the flow kernel on indexes of 65536 vectors or more for
+ *   moderate batches     up to 256 queries (2048 for k > 32) at (128, 16) and
+ *                        (128, 32), and at (96, 16) and (96, 32) for fewer than
+ *                        3072 (more on lists shorter than 500 vectors; k > 32:
+ *                        any number);
+ *   otherwise            an MFMA screen with an exact rescore (no per-(query,
+ *                        list) LUT): every query's first list gives an upper
+ *                        bound T on its k-th distance, every probed vector whose
+ *                        rigorous lower bound does not exceed T is rescored with
+ *                        the reference's direct ADC form (gpu_global.cu:259-319,
+ *                        bit-identical to the LUT sum), and the few queries it
+ *                        cannot settle (a first list shorter than k, more than
+ *                        512 candidates) go to the split LUT kernel.
+ * The screen and the split kernel need fgpu_search_workspace_bytes (the size for
+ * a large batch serves smaller ones too); a smaller workspace that still holds
+ * the coarse step runs the other LUT kernels. */
 size_t fgpu_search_workspace_bytes(int nq, int nlist, int nprobe);
 fgpu_status fgpu_search(const fgpu_index* idx, const float* d_queries, int nq, int nprobe, int k,
                         float prune_ratio, int32_t* d_out_ids, float* d_out_dists,
