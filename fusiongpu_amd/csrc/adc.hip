@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kNT) void adc_plain_kernel(AdcArgs a) {
 // split over the idle workgroups: S = grid / count parts (at most what the
 // query's part of the workspace can hold), part j walking probes j, j + S, ....
 // Every part starts from the query's bound key (the screen's rescore leaves
-// the key after the k-th best of the candidates it did keep, kNoThr without
+// the key after the k-th best of the candidates it did keep, kPadKey without
 // any; a key must be below it to enter), skips
 // the lists whose lower bound exceeds it, and shares the running k-th key with
 // the other parts through that key in global memory (a 64-bit atomic min; a
